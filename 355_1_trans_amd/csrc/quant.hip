@@ -16,11 +16,13 @@
 //     candidate_m10 host.cc:194-206).
 //
 // All of it is HBM-bound byte work: one pass over the input with 16-byte
-// loads, coalesced stores, no LDS round trips beyond the 128x128 weight
-// block's amax.  The value codecs below are written from the format
-// definitions (OCP E4M3 / E2M1, round to nearest even, saturating) so that
-// the codes are bit-identical to the host quantizers the tests compare with.
+// loads, coalesced stores; only scales go through LDS.  The value codecs
+// below are written from the format definitions (OCP E4M3 / E2M1, round to
+// nearest even, saturating); groups of ordinary magnitudes use the hardware's
+// conversions instead, which give the same codes, so all codes are
+// bit-identical to the host quantizers the tests compare with.
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -108,6 +110,171 @@ __device__ __forceinline__ float group_max(float v) {
     return v;
 }
 
+// The same over 4 or 16 lanes on bit patterns, by DPP (no LDS pipe): quad
+// permutes, then row rotations, which leave every lane of a 16-lane row with
+// the row's maximum.
+template <int WIDTH>
+__device__ __forceinline__ uint32_t group_max_bits(uint32_t v) {
+    static_assert(WIDTH == 4 || WIDTH == 16, "one quad or one DPP row");
+    auto step = [&](uint32_t o) { v = v > o ? v : o; };
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));     // quad_perm [1,0,3,2]
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));     // quad_perm [2,3,0,1]
+    if constexpr (WIDTH == 16) {
+        step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, true));    // row_ror:4
+        step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, true));    // row_ror:8
+    }
+    return v;
+}
+
+// ---------------------------------------------------------------- fast codecs
+// For a group whose |amax| is 0 or in [2^-80, inf) the codes come from the
+// gfx950 conversion instructions, which round to nearest even exactly as the
+// codecs above (all bf16 values x 207 scale exponents, all fp32 patterns up
+// to 448 compared on the GPU: no difference); other groups (infinities,
+// NaN, amax below 2^-80, where the quotient's remainder could underflow)
+// take the codecs above.  Bit patterns of |x| order like the values, and NaN
+// above infinity, so one integer maximum finds amax and both exceptions.
+constexpr uint32_t kFastLo = (127u - 80u) << 23, kInfBits = 0x7f800000u;
+__device__ __forceinline__ bool fast_group(uint32_t amax) { return amax == 0u || (amax >= kFastLo && amax < kInfBits); }
+
+// mx_exp of a fast group from the bits of amax: the smallest E with
+// amax <= qmax 2^E is amax's exponent less qmax's, one more when its
+// mantissa is above qmax's (448 = 1.75 2^8, 6 = 1.5 2^2).  mx_exp's rounded
+// quotient never crosses that line (every normal amax compared).
+template <int FMT>
+__device__ __forceinline__ int fast_exp(uint32_t amax) {
+    if (amax == 0u) return 0;
+    return FMT == 2 ? (int)((amax + 0x3fffffu) >> 23) - 129 : (int)((amax + 0x1fffffu) >> 23) - 135;
+}
+
+// x / s rounded to nearest, r = 1 / s rounded to nearest: one Newton step on
+// the quotient, whose remainder is exact (P. Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34, 1990).  The remainder is taken with its sign turned so that x =
+// -0 keeps its sign.
+__device__ __forceinline__ float div_by(float x, float s, float r) {
+    const float q = x * r;
+    return fmaf(-fmaf(q, s, -x), r, q);
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8), aligned(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+
+// Eight consecutive input elements as loaded (16 or 32 bytes; the hardware
+// takes vector loads and stores at dword, and for codes at byte, alignment).
+template <bool BF16IN>
+struct Unit;
+template <>
+struct Unit<true> {
+    i32x4 w;
+    __device__ __forceinline__ void load(const void* base, long long elem) {
+        w = __builtin_bit_cast(i32x4, *(const bf16x8*)((const uint16_t*)base + elem));
+    }
+    __device__ __forceinline__ void zero() { w = i32x4{0, 0, 0, 0}; }
+    __device__ __forceinline__ uint32_t amax_bits() const {
+        u16x2 m = {0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[i] & 0x7fff7fff));
+        return (uint32_t)(m[0] > m[1] ? m[0] : m[1]) << 16;
+    }
+    __device__ __forceinline__ float f(int i) const {
+        return __uint_as_float((i & 1) ? (uint32_t)w[i >> 1] & 0xffff0000u : (uint32_t)w[i >> 1] << 16);
+    }
+    __device__ __forceinline__ bf16x2 pair(int i) const {
+        const int d = w[i];    // a value of its own: bit-casting the vector's element in place takes element 0
+        return __builtin_bit_cast(bf16x2, d);
+    }
+    template <int I>
+    __device__ __forceinline__ i16x2 cvt8(i16x2 old, float s) const {    // pair I of the unit into half I % 2
+        return __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(old, pair(I), s, I & 1);
+    }
+    template <int I>
+    __device__ __forceinline__ uint32_t cvt4(uint32_t old, float s) const {    // pair I into byte I
+        return __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, pair(I), s, I);
+    }
+};
+template <>
+struct Unit<false> {
+    f32x4 lo, hi;
+    __device__ __forceinline__ void load(const void* base, long long elem) {
+        lo = *(const f32x4*)((const float*)base + elem);
+        hi = *(const f32x4*)((const float*)base + elem + 4);
+    }
+    __device__ __forceinline__ void zero() { lo = hi = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    __device__ __forceinline__ uint32_t amax_bits() const {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t b = __float_as_uint(f(i)) & 0x7fffffffu;
+            m = m > b ? m : b;
+        }
+        return m;
+    }
+    __device__ __forceinline__ float f(int i) const { return i < 4 ? lo[i & 3] : hi[i & 3]; }
+    template <int I>
+    __device__ __forceinline__ i16x2 cvt8(i16x2 old, float s) const {
+        return __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(old, f(2 * I), f(2 * I + 1), s, I & 1);
+    }
+    template <int I>
+    __device__ __forceinline__ uint32_t cvt4(uint32_t old, float s) const {
+        return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(old, f(2 * I), f(2 * I + 1), s, I);
+    }
+};
+
+// The codes of one unit of a fast group: FMT 0 e4m3 of x / sc (sc fp32),
+// 1 e4m3 and 2 e2m1 of x 2^-E, sc = 2^E.  Two dwords (FMT 2: one).
+template <int FMT, bool BF16IN>
+__device__ __forceinline__ u32x2 fast_codes(const Unit<BF16IN>& v, float sc) {
+    if constexpr (FMT == 0) {
+        const float r = 1.0f / sc;
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = div_by(v.f(i), sc, r);
+        int a = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false), b = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], 0, false);
+        a = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], a, true);
+        b = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], b, true);
+        return u32x2{(unsigned)a, (unsigned)b};
+    } else if constexpr (FMT == 1) {
+        i16x2 a = {0, 0}, b = {0, 0};
+        a = v.template cvt8<0>(a, sc);
+        a = v.template cvt8<1>(a, sc);
+        b = v.template cvt8<2>(b, sc);
+        b = v.template cvt8<3>(b, sc);
+        return u32x2{__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b)};
+    } else {
+        uint32_t a = v.template cvt4<0>(0u, sc);
+        a = v.template cvt4<1>(a, sc);
+        a = v.template cvt4<2>(a, sc);
+        a = v.template cvt4<3>(a, sc);
+        return u32x2{a, 0u};
+    }
+}
+
+// The same by the codecs above, for any group.
+template <int FMT, bool BF16IN>
+__device__ __forceinline__ u32x2 slow_codes(const Unit<BF16IN>& v, float sc, int E) {
+    u32x2 w = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (FMT == 0) w[i >> 2] |= f32_to_e4m3(v.f(i) / sc) << (8 * (i & 3));
+        else if constexpr (FMT == 1) w[i >> 2] |= f32_to_e4m3(__builtin_ldexpf(v.f(i), -E)) << (8 * (i & 3));
+        else w[0] |= f32_to_e2m1(__builtin_ldexpf(v.f(i), -E)) << (4 * i);
+    }
+    return w;
+}
+
+template <bool BF16IN>
+__device__ __forceinline__ float amax8(const Unit<BF16IN>& v) {
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v.f(i)));
+    return m;
+}
+
 // byte offset of (row, group) in aiter's e8m0_shuffle order (rows padded to
 // 32, groups to 8; MX4 candidate_m10 host.cc:194-206)
 __device__ __forceinline__ long long shuffled_scale_offset(int r, int g, int kg8) {
@@ -123,51 +290,117 @@ struct QuantArgs {
     long long s_sm, s_sk;    // scale element strides along rows and K blocks (row-major / column-major)
     int rows, k;
     int kg8;                 // e8m0_shuffle: K/32 rounded up to 8
+    int lc;                  // log2 of the tile's units of 8 columns
+    int ctiles;              // tiles along K
 };
 
-// Row-wise group quantizer: one thread per 4 consecutive elements, GROUP
-// elements per scale (32 for MX, 128 for the 1x128 activation blocks).
+// Row-wise group quantizer, GROUP elements per scale (32 for MX, 128 for
+// the 1x128 activation blocks).
 //   FMT  0: e4m3 with fp32 scale amax / 448 (x / scale, IEEE division)
 //        1: e4m3 with E8M0 scale 2^ceil(log2(amax / 448))
 //        2: e2m1 with E8M0 scale 2^ceil(log2(amax / 6))
 // SHUF: E8M0 scales in e8m0_shuffle order instead of (s_sm, s_sk) strides.
-template <int FMT, int GROUP, bool BF16IN, bool SHUF>
+//
+// A workgroup takes a tile of 8 << lc columns and U (256 >> lc) rows, one
+// unit of 8 elements per thread and row pass: a wave reads 1 KB (bf16) per
+// load, all U loads first.  A group's amax is 4 or 16 neighbouring lanes'
+// (one quad / DPP row).  The tile's scales meet in LDS and leave in the
+// order of their layout: whole runs of a row, of a column, or (SHUF, tiles
+// of 32 rows x 256 columns) the whole 256-byte shuffled block, whose padding
+// rows and groups are written as 0x7F here rather than by a fill before.
+//
+// Bound by HBM.  One thread per 4 elements with the codecs in software (20
+// instructions a code, 64-bit divisions for the row) was bound by its VALU
+// work instead.  Time per launch in a graph, before -> after, bf16 in:
+//   4096 x 7168   fp32 scales 37.9 -> 17.9 us (4.9 TB/s), E8M0 per 128
+//                 35.4 -> 15.7 (5.6), MXFP8 33.7 -> 15.2 (5.8), MXFP4
+//                 36.5 -> 13.7 (5.4), shuffled 39.2 -> 14.4 (5.1)
+//   7168 x 16384  MXFP4 shuffled 150 -> 43.4 us (6.8 TB/s)
+//   500 x 7168    MXFP8 6.7 -> 3.2 us
+//   32 x 7168     fp32 scales 2.9 -> 2.3 us (an empty launch takes 1.8)
+//   57 x 7168     MXFP4 shuffled, with the padding fill's launch 4.8 -> 2.4
+// fp32 in: 1.2-2.9x, 5.2-7.2 TB/s from 4096 x 2048.
+template <int FMT, int GROUP, bool BF16IN, bool SHUF, int U>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs p) {
-    constexpr int TPG = GROUP / 4;    // threads per group
-    const long long per_row = p.k / 4;
-    const long long units = (long long)p.rows * per_row;
-    for (long long u = (long long)blockIdx.x * 256 + threadIdx.x; u < units; u += (long long)gridDim.x * 256) {
-        const int r = (int)(u / per_row);
-        const int c4 = (int)(u - (long long)r * per_row);
-        const f32x4 v = load4<BF16IN>(p.x, (long long)r * p.ldx + 4 * c4);
-        const float amax = group_max<TPG>(amax4(v));
-        const int g = (4 * c4) / GROUP;
-        const bool lead = (c4 % TPG) == 0;
-        if constexpr (FMT == 0) {
-            const float sc = amax > 0.0f ? amax / 448.0f : 1.0f;
-            const uint32_t w = f32_to_e4m3(v[0] / sc) | (f32_to_e4m3(v[1] / sc) << 8) |
-                               (f32_to_e4m3(v[2] / sc) << 16) | (f32_to_e4m3(v[3] / sc) << 24);
-            *(uint32_t*)(p.q + (long long)r * p.ldq + 4 * c4) = w;
-            if (lead) ((float*)p.s)[r * p.s_sm + g * p.s_sk] = sc;
-        } else {
-            const int E = mx_exp(amax, FMT == 2 ? 6.0f : 448.0f);
-            if constexpr (FMT == 1) {
-                const uint32_t w = f32_to_e4m3(__builtin_ldexpf(v[0], -E)) |
-                                   (f32_to_e4m3(__builtin_ldexpf(v[1], -E)) << 8) |
-                                   (f32_to_e4m3(__builtin_ldexpf(v[2], -E)) << 16) |
-                                   (f32_to_e4m3(__builtin_ldexpf(v[3], -E)) << 24);
-                *(uint32_t*)(p.q + (long long)r * p.ldq + 4 * c4) = w;
+    constexpr int UPG = GROUP / 8;                 // units (lanes) per group
+    constexpr int LUPG = GROUP == 32 ? 2 : 4;
+    constexpr int NSC = U * 256 / UPG;             // scales of a tile
+    typedef typename std::conditional<FMT == 0, float, uint8_t>::type Scale;
+    __shared__ Scale sc_tile[NSC];
+    const int t = threadIdx.x, lc = p.lc;
+    const int rt = (int)(blockIdx.x / (unsigned)p.ctiles), ct = (int)(blockIdx.x - (unsigned)rt * (unsigned)p.ctiles);
+    const int rpp = 256 >> lc;                     // rows per pass
+    const long long row0 = (long long)rt * (U * rpp);
+    const int lr = t >> lc, lu = t & ((1 << lc) - 1), col = (ct << (lc + 3)) + 8 * lu;
+    const bool col_ok = col < p.k;
+    Unit<BF16IN> v[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const long long r = row0 + i * rpp + lr;
+        v[i].zero();
+        if (col_ok && r < p.rows) v[i].load(p.x, r * p.ldx + col);
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const long long r = row0 + i * rpp + lr;
+        const bool ok = col_ok && r < p.rows;
+        const uint32_t amax = group_max_bits<UPG>(v[i].amax_bits());
+        float sc = 1.0f;
+        int E = 0;
+        u32x2 w;
+        if (fast_group(amax)) {
+            if constexpr (FMT == 0) {
+                sc = amax != 0u ? __uint_as_float(amax) / 448.0f : 1.0f;
             } else {
-                const uint32_t lo = f32_to_e2m1(__builtin_ldexpf(v[0], -E)) | (f32_to_e2m1(__builtin_ldexpf(v[1], -E)) << 4);
-                const uint32_t hi = f32_to_e2m1(__builtin_ldexpf(v[2], -E)) | (f32_to_e2m1(__builtin_ldexpf(v[3], -E)) << 4);
-                *(uint16_t*)(p.q + (long long)r * p.ldq + 2 * c4) = (uint16_t)(lo | (hi << 8));
+                E = fast_exp<FMT>(amax);
+                sc = __uint_as_float((uint32_t)(E + 127) << 23);
             }
-            if (lead) {
-                uint8_t* e = (uint8_t*)p.s;
-                const long long off = SHUF ? shuffled_scale_offset(r, g, p.kg8) : r * p.s_sm + g * p.s_sk;
-                e[off] = (uint8_t)(E + 127);
-            }
+            w = fast_codes<FMT, BF16IN>(v[i], sc);
+        } else {
+            const float am = group_max<UPG>(amax8<BF16IN>(v[i]));
+            if constexpr (FMT == 0) sc = am > 0.0f ? am / 448.0f : 1.0f;
+            else E = mx_exp(am, FMT == 2 ? 6.0f : 448.0f);
+            w = slow_codes<FMT, BF16IN>(v[i], sc, E);
         }
+        if (ok) {
+            uint8_t* q = p.q + r * p.ldq + (FMT == 2 ? col >> 1 : col);
+            if constexpr (FMT == 2) *(u32_a2*)q = w[0];
+            else *(u32x2_a4*)q = __builtin_bit_cast(u32x2_a4, w);
+        }
+        if ((lu & (UPG - 1)) == 0) {
+            Scale o;
+            if constexpr (FMT == 0) o = sc;
+            else o = SHUF && !ok ? (uint8_t)0x7f : (uint8_t)(E + 127);
+            sc_tile[((i * rpp + lr) << (lc - LUPG)) + (lu >> LUPG)] = o;
+        }
+    }
+    __syncthreads();
+    const int lg = lc - LUPG, g0 = ct << lg;       // log2 of the tile's groups per row; its first group
+    if (t >= NSC) return;
+    if constexpr (SHUF) {
+        // padding included: rows to a multiple of 32, groups to one of 8
+        int r, g;
+        if constexpr (U == 4) {                    // e = byte of the tile's one shuffled block
+            r = (t & 1) * 16 + ((t & 63) >> 2);
+            g = ((t & 3) >> 1) * 4 + (t >> 6);
+        } else {
+            r = t >> lg;
+            g = t & ((1 << lg) - 1);
+        }
+        if (row0 + r < (p.rows + 31LL) / 32 * 32 && g0 + g < p.kg8)
+            ((uint8_t*)p.s)[shuffled_scale_offset((int)(row0 + r), g0 + g, p.kg8)] = sc_tile[(r << lg) + g];
+    } else {
+        const int lrows = 8 - lc + (U == 4 ? 2 : 0);
+        int r, g;
+        if (p.s_sk == 1) {                         // a row's groups are neighbours
+            r = t >> lg;
+            g = t & ((1 << lg) - 1);
+        } else {                                   // a group's rows are neighbours
+            g = t >> lrows;
+            r = t & ((1 << lrows) - 1);
+        }
+        if (row0 + r < p.rows && g0 + g < p.k / GROUP)
+            ((Scale*)p.s)[(row0 + r) * p.s_sm + (g0 + g) * p.s_sk] = sc_tile[(r << lg) + g];
     }
 }
 
@@ -219,12 +452,6 @@ __global__ __launch_bounds__(256) void quant_wgt_block_kernel(const QuantArgs p)
                     (f32_to_e4m3(__builtin_ldexpf(v[i][3], -E)) << 24);
         }
     }
-}
-
-// bytes := 0x7F (E8M0 1.0), the padding value of e8m0_shuffle
-__global__ __launch_bounds__(256) void fill_7f_kernel(uint8_t* dst, long long bytes) {
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < bytes; i += (long long)gridDim.x * 256)
-        dst[i] = 0x7f;
 }
 
 // ---------------------------------------------------------------- layouts
@@ -322,6 +549,10 @@ __global__ __launch_bounds__(256) void e8m0_shuffle_blocks_kernel(const ShuffleA
         i32x4{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
 }
 
+// Row passes of 256 threads up to which the row quantizer runs one per
+// workgroup: 2048 workgroups are one round of the chip at eight per CU.
+constexpr long long kQuantOnePass = 2048;
+
 unsigned grid_for(long long units) {
     const long long b = (units + 255) / 256;
     return (unsigned)(b < 8192 ? (b > 0 ? b : 1) : 8192);
@@ -344,17 +575,28 @@ hipError_t launch_quant_rows(int fmt, int group, bool bf16in, bool shuffle, cons
     p.rows = rows;
     p.k = k;
     p.kg8 = (k / 32 + 7) / 8 * 8;
-    const unsigned grid = grid_for((long long)rows * (k / 4));
-    if (shuffle) {
-        const long long bytes = (long long)(rows + 31) / 32 * 32 * p.kg8;
-        if (rows % 32 || (k / 32) % 8) {
-            fill_7f_kernel<<<grid_for(bytes), 256, 0, st>>>((uint8_t*)s, bytes);
-            trace_launch("fill_7f");
-        }
-    }
+    // Tile: scales that run along K (row-major) take up to 1024 columns, so
+    // a row's scales leave in runs of 8 floats or 32 bytes; column-major and
+    // shuffled scales take 256 columns of 32 rows.  Narrow K takes a
+    // narrower tile (no idle columns).  One row pass per workgroup while
+    // that leaves the chip room (latency counts, not bytes per workgroup),
+    // else four.
+    const bool tall = shuffle || s_sk != 1;
+    int lc = tall ? 5 : 7;
+    while (!shuffle && lc > (group == 32 ? 2 : 4) && (4LL << lc) >= k) --lc;
+    p.lc = lc;
+    p.ctiles = (k + (8 << lc) - 1) / (8 << lc);
+    const long long prow = shuffle ? (rows + 31LL) / 32 * 32 : rows;
+    const long long passes = (prow + (256 >> lc) - 1) / (256 >> lc) * p.ctiles;
+    const bool one = passes <= kQuantOnePass;
+    const long long rpt = (256 >> lc) * (one ? 1 : 4);
+    const long long blocks = (prow + rpt - 1) / rpt * p.ctiles;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    const unsigned grid = (unsigned)blocks;
 #define QG_QUANT(F, G, B, S)                                                                            \
     if (fmt == F && group == G && bf16in == B && shuffle == S) {                                        \
-        quant_rows_kernel<F, G, B, S><<<grid, 256, 0, st>>>(p);                                         \
+        if (one) quant_rows_kernel<F, G, B, S, 1><<<grid, 256, 0, st>>>(p);                             \
+        else quant_rows_kernel<F, G, B, S, 4><<<grid, 256, 0, st>>>(p);                                 \
         trace_launch("quant_rows<%s,g%d,%s%s>", F == 0 ? "e4m3,fp32" : F == 1 ? "e4m3,e8m0" : "e2m1,e8m0", G, \
                      B ? "bf16" : "fp32", S ? ",shuffled" : "");                                        \
         return hipGetLastError();                                                                       \

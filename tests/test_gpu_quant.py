@@ -165,6 +165,64 @@ def test_quant_extreme_magnitudes(qgemm, gpu):
     assert np.array_equal(s.cpu().numpy().view(np.uint32), sr.view(np.uint32))
 
 
+# Tile edges of the row quantizers: one and four row passes per workgroup,
+# narrow, ragged and wide K, rows and columns past the last tile, shuffled
+# padding -- with rows of -0, of zeros, infinities and NaN, and amax at and
+# around 2^-80, on sources whose rows are 8-byte (bf16) aligned only.
+@pytest.mark.parametrize("rows,k", [(1, 32), (9, 128), (31, 224), (33, 1152), (257, 96), (1030, 2080), (2100, 1024),
+                                    (70000, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quant_rows_tile_edges_and_exceptions(qgemm, gpu, rows, k, dtype):
+    x = O.randn((rows, k), rows + k, 3)
+    if rows > 8:
+        x[1] = 0.0
+        x[2, ::3] = -0.0
+        x[3, 5], x[4, 7], x[5, 9] = np.inf, -np.inf, np.nan
+        x[6] = np.clip(x[6], -1, 1) * np.float32(2.0 ** -80)
+        x[6, 0] = np.float32(2.0 ** -80)                      # the smallest amax of the conversion path
+        x[7] = np.clip(x[7], -0.99, 0.99) * np.float32(2.0 ** -80)
+        x[8] *= np.float32(2.0 ** 125)
+    ref = x if dtype == torch.float32 else _bf16_round(x)
+    flat = torch.empty(rows * (k + 4) + 4, dtype=dtype, device=gpu)
+    src = flat[4:].view(rows, k + 4)[:, :k]
+    src.copy_(torch.from_numpy(ref).to(dtype).to(gpu))     # rounded on the host, NaN and all
+
+    def same(got, want):
+        got = got.view(torch.uint8).cpu().numpy()
+        nan = (want & 0x7F) == 0x7F                           # a NaN's sign is not specified
+        assert np.array_equal(np.where(nan, got & 0x7F, got), np.where(nan, want & 0x7F, want))
+
+    def infinite_groups(q, e, group, top):
+        """A group with an infinity has the top exponent, which takes every finite value to 0 and the infinity to the
+        top code (the host recipe leaves the exponent of an infinity open)."""
+        bad = np.isinf(ref).reshape(rows, -1, group).any(-1)
+        e[bad] = 254
+        sign = np.where(np.signbit(ref), 8 if top == 7 else 128, 0)
+        codes = np.where(np.isinf(ref), top, 0) | sign
+        if top == 7:
+            codes = codes[:, ::2] | codes[:, 1::2] << 4
+        wide = np.repeat(bad, group // (2 if top == 7 else 1), axis=1)
+        return np.where(wide, codes, q).astype(np.uint8), e
+
+    with np.errstate(all="ignore"):
+        for fn, ofn, top in ((qgemm.quant_mxfp8, O.quant_mx8, 0x7E), (qgemm.quant_mxfp4, O.quant_mx4, 7)):
+            qr, er = infinite_groups(*ofn(ref), 32, top)
+            for shuffle in (False, True):
+                q, e = fn(src, shuffle=shuffle)
+                same(q, qr) if fn is qgemm.quant_mxfp8 else np.testing.assert_array_equal(q.cpu().numpy(), qr)
+                assert np.array_equal(e.cpu().numpy(), O.e8m0_shuffle(er) if shuffle else er)
+        if k % 128 == 0:
+            qr, sr = O.quant_bs_act(ref)
+            for layout in ("mk", "km"):
+                q, s = qgemm.quant_fp8_blockscale(src, "1x128", layout)
+                same(q, qr)
+                assert np.array_equal(s.cpu().numpy().view(np.uint32), sr.view(np.uint32))
+            qr, er = infinite_groups(*O.quant_bs_e8m0_act(ref), 128, 0x7E)
+            q, e = qgemm.quant_fp8_e8m0_blockscale(src, "1x128")
+            same(q, qr)
+            assert np.array_equal(e.cpu().numpy(), er)
+
+
 # ----------------------------------------------------------------- layouts
 @pytest.mark.parametrize("n,k", [(48, 384), (7168, 512), (37, 256)])
 def test_device_layouts_match_host(qgemm, gpu, n, k):
