@@ -86,22 +86,6 @@ __device__ __forceinline__ int mx_exp(float amax, float qmax) {
     return e < -127 ? -127 : (e > 127 ? 127 : e);
 }
 
-// Four consecutive input elements as fp32 (bf16 widens exactly).
-template <bool BF16IN>
-__device__ __forceinline__ f32x4 load4(const void* base, long long elem) {
-    if constexpr (BF16IN) {
-        const uint2 v = *(const uint2*)((const uint16_t*)base + elem);
-        return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
-                     __uint_as_float(v.y & 0xffff0000u)};
-    } else {
-        return *(const f32x4*)((const float*)base + elem);
-    }
-}
-
-__device__ __forceinline__ float amax4(f32x4 v) {
-    return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-}
-
 // max over `width` consecutive lanes (width a power of two <= 64)
 template <int WIDTH>
 __device__ __forceinline__ float group_max(float v) {
@@ -405,51 +389,72 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs p) {
 }
 
 // 128 x 128 weight-block quantizer: one workgroup (4 waves) per block;
-// thread t holds columns 4(t % 32) .. +3 of rows t/32 + 8i (i < 16) -- each
-// load instruction covers two whole 512-byte rows -- then the block's amax
-// meets in LDS.  Rows past N belong to no block element (masked).
+// thread t holds columns 8(t % 16) .. +7 of rows t/16 + 16i (i < 8) -- each
+// load instruction covers four whole 256-byte (bf16) rows of the block -- and
+// the block's amax meets in LDS.  Rows past N belong to no block element
+// (masked).  Codes as in the row quantizers; the whole workgroup takes the
+// software codecs when the block holds an infinity, NaN or a tiny amax.
 //   FMT 0: fp32 scale amax / 448; 1: E8M0 2^ceil(log2(amax / 448)).
+// HBM-bound.  Four columns per thread and the software codecs -> this, per
+// launch in a graph, bf16 in, fp32 / E8M0 scales: 192 x 2048 14.9 / 13.2 ->
+// 3.6 / 3.1 us, 4096 x 7168 39.8 / 35.8 -> 14.9 / 14.6 (5.9 TB/s),
+// 7168 x 16384 143 / 132 -> 63 / 63; fp32 in 1.05-3.6x (5.3-6.8 TB/s).
 template <int FMT, bool BF16IN>
 __global__ __launch_bounds__(256) void quant_wgt_block_kernel(const QuantArgs p) {
-    __shared__ float wmax[4];
+    __shared__ uint32_t wmax[8];
     const int g = blockIdx.x, nb = blockIdx.y, t = threadIdx.x;
-    const int c4 = t & 31, r0 = t >> 5;
+    const int col = g * 128 + 8 * (t & 15), r0 = t >> 4;
     const int rows = min(128, p.rows - nb * 128);
-    f32x4 v[16];
-    float amax = 0.0f;
+    Unit<BF16IN> v[8];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int r = r0 + 8 * i;
-        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (r < rows) v[i] = load4<BF16IN>(p.x, (long long)(nb * 128 + r) * p.ldx + g * 128 + 4 * c4);
-        amax = fmaxf(amax, amax4(v[i]));
+    for (int i = 0; i < 8; ++i) {
+        const int r = r0 + 16 * i;
+        v[i].zero();
+        if (r < rows) v[i].load(p.x, (long long)(nb * 128 + r) * p.ldx + col);
     }
-    amax = group_max<64>(amax);
-    if ((t & 63) == 0) wmax[t >> 6] = amax;
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t b = v[i].amax_bits();
+        bits = bits > b ? bits : b;
+    }
+    bits = group_max_bits<16>(bits);
+#pragma unroll
+    for (int d = 16; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)bits, d, 64);
+        bits = bits > o ? bits : o;
+    }
+    if ((t & 63) == 0) wmax[t >> 6] = bits;
     __syncthreads();
-    amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    bits = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    const bool fast = fast_group(bits);
+    float amax = __uint_as_float(bits);
+    if (!fast) {                                   // NaN does not count towards amax
+        amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, amax8<BF16IN>(v[i]));
+        amax = group_max<64>(amax);
+        if ((t & 63) == 0) wmax[4 + (t >> 6)] = __float_as_uint(amax);
+        __syncthreads();
+        amax = fmaxf(fmaxf(__uint_as_float(wmax[4]), __uint_as_float(wmax[5])),
+                     fmaxf(__uint_as_float(wmax[6]), __uint_as_float(wmax[7])));
+    }
+    float sc = 1.0f;
+    int E = 0;
     if constexpr (FMT == 0) {
-        const float sc = amax > 0.0f ? amax / 448.0f : 1.0f;
+        sc = amax > 0.0f ? amax / 448.0f : 1.0f;
         if (t == 0) ((float*)p.s)[nb * p.s_sm + g] = sc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = r0 + 8 * i;
-            if (r < rows)
-                *(uint32_t*)(p.q + (long long)(nb * 128 + r) * p.ldq + g * 128 + 4 * c4) =
-                    f32_to_e4m3(v[i][0] / sc) | (f32_to_e4m3(v[i][1] / sc) << 8) |
-                    (f32_to_e4m3(v[i][2] / sc) << 16) | (f32_to_e4m3(v[i][3] / sc) << 24);
-        }
     } else {
-        const int E = mx_exp(amax, 448.0f);
+        E = mx_exp(amax, 448.0f);
         if (t == 0) ((uint8_t*)p.s)[nb * p.s_sm + g] = (uint8_t)(E + 127);
+        if (fast) sc = __uint_as_float((uint32_t)(E + 127) << 23);
+    }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = r0 + 8 * i;
-            if (r < rows)
-                *(uint32_t*)(p.q + (long long)(nb * 128 + r) * p.ldq + g * 128 + 4 * c4) =
-                    f32_to_e4m3(__builtin_ldexpf(v[i][0], -E)) | (f32_to_e4m3(__builtin_ldexpf(v[i][1], -E)) << 8) |
-                    (f32_to_e4m3(__builtin_ldexpf(v[i][2], -E)) << 16) |
-                    (f32_to_e4m3(__builtin_ldexpf(v[i][3], -E)) << 24);
+    for (int i = 0; i < 8; ++i) {
+        const int r = r0 + 16 * i;
+        if (r < rows) {
+            const u32x2 w = fast ? fast_codes<FMT, BF16IN>(v[i], sc) : slow_codes<FMT, BF16IN>(v[i], sc, E);
+            *(u32x2_a4*)(p.q + (long long)(nb * 128 + r) * p.ldq + col) = __builtin_bit_cast(u32x2_a4, w);
         }
     }
 }

@@ -56,6 +56,32 @@ def test_quant_fp8_blockscale_wgt(qgemm, gpu, n, k, dtype):
     assert np.array_equal(s.cpu().numpy().view(np.uint32), sr.view(np.uint32))
 
 
+@pytest.mark.parametrize("n,k", [(1, 128), (130, 384), (1024, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quant_wgt_block_exceptions(qgemm, gpu, n, k, dtype):
+    """Blocks with a NaN, a tiny or a huge amax, all zeros and -0, partial last blocks, 8-byte (bf16) aligned rows."""
+    x = O.randn((n, k), n + k, 4)
+    for b, scale in enumerate((2.0 ** -80, 2.0 ** -81, 2.0 ** 124, 0.0, -0.0)):
+        blk = x[128 * b:128 * (b + 1), :128]
+        blk *= np.float32(scale)
+    x[n // 2, -1] = np.nan
+    ref = x if dtype == torch.float32 else _bf16_round(x)
+    flat = torch.empty(n * (k + 4) + 4, dtype=dtype, device=gpu)
+    src = flat[4:].view(n, k + 4)[:, :k]
+    src.copy_(torch.from_numpy(ref).to(dtype).to(gpu))
+    qr, sr = O.quant_bs_wgt(ref)
+    q, s = qgemm.quant_fp8_blockscale(src, "128x128")
+    nan = (qr & 0x7F) == 0x7F                                 # a NaN's sign is not specified
+    got = q.view(torch.uint8).cpu().numpy()
+    assert np.array_equal(np.where(nan, got & 0x7F, got), np.where(nan, qr & 0x7F, qr))
+    assert np.array_equal(s.cpu().numpy().view(np.uint32), sr.view(np.uint32))
+    qr, er = O.quant_bs_e8m0_wgt(ref)
+    q, e = qgemm.quant_fp8_e8m0_blockscale(src, "128x128")
+    got = q.view(torch.uint8).cpu().numpy()
+    assert np.array_equal(np.where(nan, got & 0x7F, got), np.where(nan, qr & 0x7F, qr))
+    assert np.array_equal(e.cpu().numpy(), er)
+
+
 @pytest.mark.parametrize("rows,k", [(300, 4096), (8, 1024)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_quant_fp8_e8m0(qgemm, gpu, rows, k, dtype):
