@@ -377,6 +377,10 @@ void plan_mid(Plan& p, int m, int n, int k_tiles, int batch, int cus, bool force
         split = std::max<long long>(split, std::min<long long>(cus / tiles, k_tiles / kMidMinKtDeep));
     if (split <= 1) return;
     p.kt_per_split = ceil_div(k_tiles, (int)split);
+    // more workgroups than CUs run the two-stage form, which moves its scales
+    // in panels of four K-tiles only when its slices start on one
+    if (tiles * ceil_div(k_tiles, p.kt_per_split) > cus && k_tiles % 4 == 0)
+        p.kt_per_split = ceil_div(p.kt_per_split, 4) * 4;
     p.splitk = ceil_div(k_tiles, p.kt_per_split);
     if (p.splitk > 1) {
         p.ctr_bytes = kCounterBytes;    // unused by this kernel: keeps the partials past the counter block

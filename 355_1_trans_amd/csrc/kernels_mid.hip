@@ -9,8 +9,14 @@ namespace qg {
 
 template <BLay BL, int ST, ScaleKind SK, int FMT, bool NTB = false>
 static void mid_go(const MidArgs& a, const dim3& grid, bool bf16, hipStream_t s) {
-    if (bf16) mid_gemm_kernel<true, BL, ST, SK, FMT, NTB><<<grid, 256, 0, s>>>(a);
-    else mid_gemm_kernel<false, BL, ST, SK, FMT, NTB><<<grid, 256, 0, s>>>(a);
+    const int threads = ST == 2 ? 256 : 512;
+    if (a.panels) {
+        if (bf16) mid_gemm_kernel<true, BL, ST, SK, FMT, NTB, true><<<grid, threads, 0, s>>>(a);
+        else mid_gemm_kernel<false, BL, ST, SK, FMT, NTB, true><<<grid, threads, 0, s>>>(a);
+    } else {
+        if (bf16) mid_gemm_kernel<true, BL, ST, SK, FMT, NTB><<<grid, threads, 0, s>>>(a);
+        else mid_gemm_kernel<false, BL, ST, SK, FMT, NTB><<<grid, threads, 0, s>>>(a);
+    }
     trace_launch("mid_gemm<%s,%s,%s,%s,st%d%s,splitk%d>", FMT == kFmtFp4 ? "fp4" : "fp8", scale_name(SK),
                  layout_name(BL), bf16 ? "bf16" : "fp32", ST, NTB ? ",ntb" : "", (int)grid.y);
 }
@@ -54,7 +60,25 @@ hipError_t launch_splitk_reduce(const SplitReduceArgs& r, bool bf16, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_mid(const MidArgs& a, int batch, bool bf16, MidKind kind, int stages, hipStream_t s) {
+// Whether the scales can move as 4-K-tile panels: rows of whole panels, 16
+// bytes (fp4: 32) of consecutive K per row, 16-byte aligned; in the two-stage
+// form slices that start on a panel.  (Column-major fp32 scales are 64
+// consecutive floats per DMA already.)
+static bool mid_panels(const MidArgs& a, int batch, MidKind kind, int stages) {
+    const TileArgs& t = a.t;
+    const bool mx = kind == MidKind::MX8 || kind == MidKind::MX4;
+    const int nkt = t.kbytes / 128;
+    if (nkt % 4 || (stages == 2 && a.splitk > 1 && a.kt_per_split % 4)) return false;
+    if (!mx && t.sfa_sk != 1) return false;
+    const long long unit = mx ? 16 : 4;    // scale elements of 16 bytes
+    if (t.sfa_sm % unit || t.sfb_sn % unit) return false;
+    if (batch > 1 && (t.sfa_batch % unit || t.sfb_batch % unit)) return false;
+    return (reinterpret_cast<uintptr_t>(t.sfa) | reinterpret_cast<uintptr_t>(t.sfb)) % 16 == 0;
+}
+
+hipError_t launch_mid(const MidArgs& args, int batch, bool bf16, MidKind kind, int stages, hipStream_t s) {
+    MidArgs a = args;
+    a.panels = mid_panels(a, batch, kind, stages);
     const dim3 grid(a.t.tiles_m * a.t.tiles_n, a.splitk, batch);
     if (stages == 2) mid_kind<2>(a, grid, bf16, kind, s);
     else if (stages == 4) mid_kind<4>(a, grid, bf16, kind, s);

@@ -3,31 +3,51 @@
 //
 // At M ~ 256-4096 with narrow N the 256 x 256 tiles of bsf32_gemm.hpp leave
 // most of the 256 CUs idle (M = 1024, N = 2112: 36 tiles).  This kernel cuts
-// the tile to 128 x 128 (4 x the tiles) and can split K over workgroups; a
-// workgroup is 4 waves (one per SIMD) and two workgroups share a CU (66 KB of
-// LDS each), so one workgroup's barrier and DMA waits are covered by the
-// other's MFMAs.
+// the tile to 128 x 128 (4 x the tiles) and can split K over workgroups.
 //
-//  * wave (wm, wn) = (w / 2, w % 2) owns 64 x 64 outputs: 4 x 4 blocks of
-//    v_mfma_f32_16x16x128_f8f6f4 (unscaled fp8; one instruction = one
-//    128-deep K-tile = one scale block), 64 VGPR accumulators, each
+//  * wave (wm, wn) = (w / 2, w % 2) of four owns 64 x 64 outputs: 4 x 4
+//    blocks of v_mfma_f32_16x16x128_f8f6f4 (unscaled fp8; one instruction =
+//    one 128-deep K-tile = one scale block), 64 VGPR accumulators, each
 //    partial rescaled acc += part * (sa * sb) after the next MFMA issued;
-//  * two LDS stages of one K-tile (A 128 rows, B 128 rows, the K-tile's
-//    scales), one barrier per K-tile; the 9 DMAs per wave of K-tile t+1
-//    (buffer_load ... lds, 4 A, 4 B, 1 scale) go into the other stage,
-//    spread over K-tile t's MFMAs; DMAs past the slice use an empty-range
-//    descriptor (no branches, so the compiler's DMA waits stay exact; the
-//    loop is unrolled by two so every stage is its own LDS object);
+//  * operands move global -> LDS by DMA (buffer_load ... lds, per K-tile 4 A,
+//    4 B and the scales per wave), one barrier per K-tile; a wave's LDS reads
+//    run under its MFMAs, across the K-tile boundary too;
+//  * up to one workgroup per CU (STAGES = 4): four K-tiles in LDS and four
+//    more waves that only issue DMAs, so a DMA the texture path cannot queue
+//    does not hold up the MFMAs of the wave that issued it.  With every wave
+//    doing both, and each K-tile's first LDS reads behind its own barrier, a
+//    wave -- alone on its SIMD -- spent 42% of its cycles at waits and 27% on
+//    blocked issues;
+//  * more workgroups than CUs (STAGES = 2): two per CU (two stages each), one
+//    workgroup's barrier and DMA waits covered by the other's MFMAs; the
+//    waves issue their own DMAs, every LDS stage its own object so that the
+//    compiler's DMA waits stay exact, DMAs past the slice through an
+//    empty-range descriptor;
 //  * B' (K-panel): the tile's 128 rows of a K-tile are 16 contiguous KB;
 //    B'' (the LDS-bypass entry's fragment order): 8 blocks of 2 KB, copied
 //    as is and read back linearly (the block is the MFMA operand order);
-//  * MX (row-major B, its rows DMA'd like A's): the K-tile's E8M0 bytes of
-//    the tile's 128 A and 128 B rows ride in the stage beside the operands
-//    (4 bytes per row for fp8, 8 for fp4; one or two dword DMAs per wave)
-//    and the scaled MFMA applies them, accumulating in place (no VALU
-//    rescale).  fp8: lane (q, r) holds chunks q and q + 4 of row r with
-//    scale byte q; fp4: two MFMAs per K-tile, chunks 2q and 2q + 1 with
-//    scale bytes 2q and 2q + 1 (op_sel 0 and 1 of one 16-bit read);
+//  * MX (row-major B, its rows DMA'd like A's): the scaled MFMA applies the
+//    E8M0 bytes, accumulating in place (no VALU rescale).  fp8: lane (q, r)
+//    holds chunks q and q + 4 of row r with scale byte q; fp4: two MFMAs per
+//    K-tile, chunks 2q and 2q + 1 with scale bytes 2q and 2q + 1 (op_sel 0
+//    and 1 of one 16-bit read);
+//  * scales: row-major scales put every row's bytes of a K-tile on a cache
+//    line of its own, so a K-tile's dword DMAs (fp8 256 lines, fp4 512) cost
+//    the texture path half as much as, or as much as, its 32 KB of operands.
+//    PANEL moves four K-tiles' scales of a row at once (16 bytes, fp4 32),
+//    into one of two LDS panels, with the panel's first K-tile.
+//
+// What bounds it: an L2-resident DMA stream runs 107 GB/s per CU (32 KB in
+// 0.31 us) whatever its depth; this K loop takes 0.5 us per K-tile, and a
+// launch ~5 us around it (dispatch, the first loads, the C or partial
+// stores).  Before -> after (both forms, graph replays over rotating
+// weights): MXFP8 M = 500, N = 4096, K = 7168 37.3 -> 28.9 us, M = 128,
+// N = 7168, K = 16384 53.8 -> 36.1, MXFP4 33.7 -> 26.1, MXFP8 M = 512,
+// N = 7168, K = 2048 16.6 -> 13.3; fp32 scales M = 192, N = 7168, K = 2048
+// 15.0 -> 13.4, M = 256, K = 16384 59.3 -> 50.8; two-stage MXFP8 M = 2048,
+// N = 1536, K = 7168 51 -> 40.  1.17x geomean over 22 shapes, none slower,
+// the same bits.
+//
 //  * split-K: every workgroup stores its fp32 partial tile and returns;
 //    splitk_reduce_kernel, launched next on the stream, adds the slices in
 //    slice order (deterministic) over the whole chip.  A last-arriving
@@ -47,6 +67,7 @@ struct MidArgs {
     TileArgs t;            // tiles_m / tiles_n count 128 x 128 tiles
     float* ws;             // fp32 partials [splitk][batch][M][N] (splitk > 1)
     int splitk, kt_per_split;
+    int panels;            // scales in 4-K-tile panels (launch_mid decides)
 };
 
 // Sums the fp32 partials [splitk][batch][M][N] in slice order into C (row
@@ -136,12 +157,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 // SK = BSF32: fp8, fp32 block scales, B' or B''; SK = MX: fp8 or fp4 (FMT),
 // E8M0 scales per 32 K, row-major B, the scales applied by the MFMA.
 // NTB: B through the nontemporal cache policy (one M tile: B is read once)
-template <bool BF16, BLay BL, int STAGES, ScaleKind SK = ScaleKind::BSF32, int FMT = kFmtFp8, bool NTB = false>
-__global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(const MidArgs mp) {
+// PANEL: scales in panels of four K-tiles (see above)
+template <bool BF16, BLay BL, int STAGES, ScaleKind SK = ScaleKind::BSF32, int FMT = kFmtFp8, bool NTB = false,
+          bool PANEL = false>
+__global__ __launch_bounds__(STAGES == 2 ? 256 : 512, 2) void mid_gemm_kernel(const MidArgs mp) {
     static_assert(STAGES == 2 || STAGES == 4, "two stages (two workgroups per CU) or four (one)");
+    constexpr bool SPEC = STAGES == 4;         // four MFMA waves and four DMA waves
     constexpr bool MX = (SK == ScaleKind::MX);
     constexpr bool FP4 = (FMT == kFmtFp4);
-    static_assert(MX ? BL == BLay::RAW : (BL == BLay::KPANEL || BL == BLay::FRAG && !FP4),
+    static_assert(MX ? BL == BLay::RAW : (!FP4 && (BL == BLay::KPANEL || BL == BLay::FRAG)),
                   "MX: row-major B; fp32 block scales: fp8 with K-panel B' or fragment-order B''");
     constexpr bool FRAG = (BL == BLay::FRAG);
     constexpr bool RAW = (BL == BLay::RAW);
@@ -150,14 +174,22 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
     constexpr int KTB = MX ? (FP4 ? 8 : 4) : 4;   // scale bytes per row and K-tile (MX)
     constexpr int SA_OFF = 2 * OPB;            // BSF32: 128 fp32 row scales; MX: [128][KTB] of A
     constexpr int SB_OFF = SA_OFF + (MX ? 128 * KTB : 512);   // BSF32: 2 slots of 256 B; MX: [128][KTB] of B
-    constexpr int STAGE = SB_OFF + (MX ? 128 * KTB : 512);
-    constexpr int SCD = MX && FP4 ? 2 : 1;     // scale DMAs per wave and K-tile
-    constexpr int NDMA = 8 + SCD;              // DMAs per wave and K-tile
+    constexpr int STAGE = PANEL ? SA_OFF : SB_OFF + (MX ? 128 * KTB : 512);
+    constexpr int SCD = MX && FP4 ? 2 : 1;     // scale DMAs per wave: per K-tile, or per panel
+    // PANEL: [256 rows: A then B][4 K-tiles' bytes]; BSF32: A's 128 rows of 4 floats, then B's 4 floats, copied
+    // to every 16 bytes of 2 KB (waves 2 and 3 move what waves 0 and 1 do)
+    constexpr int PROW = MX ? 4 * KTB : 16;
+    constexpr int PAN = PANEL ? 256 * PROW : 1;
+    // DMAs per wave of K-tile y (counted from the slice's first)
+    auto ndma = [](int y) constexpr { return 8 + (PANEL ? (y % 4 == 0 ? SCD : 0) : SCD); };
 
-    __shared__ __attribute__((aligned(1024))) uint8_t st0[STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t st1[STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t st2[STAGES > 2 ? STAGE : 1];
-    __shared__ __attribute__((aligned(1024))) uint8_t st3[STAGES > 2 ? STAGE : 1];
+    // SPEC: one ring (the waves that read it issue no DMAs, so the compiler
+    // has no DMA waits to place); else one LDS object per stage and panel,
+    // which keeps those waits exact
+    __shared__ __attribute__((aligned(1024))) uint8_t st0[SPEC ? 4 * STAGE : STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t st1[SPEC ? 1 : STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t pn0[SPEC ? 2 * PAN : PAN];
+    __shared__ __attribute__((aligned(1024))) uint8_t pn1[SPEC ? 1 : PAN];
 
     const TileArgs& p = mp.t;
     // ---- tile coordinates: XCD-contiguous remap, then grouped raster ----
@@ -171,7 +203,6 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
     const int within = bid - gi * gfull;
     const int tm = first_m + within % gm;
     const int tn = within / gm;
-    const int tile = tm * p.tiles_n + tn;
     const int sk = blockIdx.y, bz = blockIdx.z;
     const int m0 = tm * BT, n0 = tn * BT;
 
@@ -182,7 +213,7 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
     const int nk = min(NKT, kt0 + mp.kt_per_split) - kt0;    // K-tiles of this slice
 
     const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), L = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane((tid >> 6) & 3), L = tid & 63;    // of the MFMA or the DMA waves
     const int wm = w >> 1, wn = w & 1;
     const int q = L >> 4, l16 = L & 15;
 
@@ -220,6 +251,8 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
     // scale block).  MX -- waves 0, 1 the K-tile's E8M0 bytes of A rows
     // [64w, 64w + 64), waves 2, 3 those of B rows [64(w-2), +64): KTB bytes
     // per row, one dword per lane (fp4: two DMAs of 32 rows)
+    // PANEL: the same rows (MX: and waves), 4 K-tiles of scales per row: 16 or
+    // (fp4) 32 bytes, one or two lanes each
     const bool sc_is_a = w < 2;
     const uint8_t* sc_base;
     int sc_voff[SCD], sc_dst[SCD];
@@ -234,25 +267,26 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
             const int row = FP4 ? r64 + 32 * s2 + (L >> 1) : r64 + L;
             const int sm = sc_is_a ? SFA_SM : SFB_SN;
             const int lim = sc_is_a ? M - 1 - m0 : N - 1 - n0;
-            sc_voff[s2] = min(row, lim) * sm + (FP4 ? (L & 1) * 4 : 0);
-            sc_dst[s2] = (sc_is_a ? SA_OFF : SB_OFF) + (FP4 ? (r64 + 32 * s2) * 8 : r64 * 4);
+            sc_voff[s2] = min(row, lim) * sm + (FP4 ? (L & 1) * (PANEL ? 16 : 4) : 0);
+            if constexpr (PANEL) sc_dst[s2] = (64 * w + 32 * s2) * PROW;
+            else sc_dst[s2] = (sc_is_a ? SA_OFF : SB_OFF) + (FP4 ? (r64 + 32 * s2) * 8 : r64 * 4);
         }
     } else {
         sc_base = sc_is_a ? SFA + 4ll * m0 * SFA_SM + 4ll * kt0 * SFA_SK
                           : SFB + 4ll * min(n0 >> 7, (N - 1) >> 7) * SFB_SN + 4ll * kt0;
         sc_voff[0] = sc_is_a ? 4 * (min(m0 + 64 * w + L, M - 1) - m0) * SFA_SM : 0;
         sc_kstep = sc_is_a ? 4ll * SFA_SK : 4ll;
-        sc_dst[0] = sc_is_a ? SA_OFF + 256 * w : SB_OFF + 256 * (w - 2);
+        if constexpr (PANEL) sc_dst[0] = 1024 * w;
+        else sc_dst[0] = sc_is_a ? SA_OFF + 256 * w : SB_OFF + 256 * (w - 2);
     }
 
     QG_LDS uint8_t* const pS0 = (QG_LDS uint8_t*)st0;
     QG_LDS uint8_t* const pS1 = (QG_LDS uint8_t*)st1;
-    QG_LDS uint8_t* const pS2 = (QG_LDS uint8_t*)st2;
-    QG_LDS uint8_t* const pS3 = (QG_LDS uint8_t*)st3;
-    auto stage = [&](auto SC) __attribute__((always_inline)) {
-        constexpr int S = decltype(SC)::value % STAGES;
-        return S == 0 ? pS0 : (S == 1 ? pS1 : (S == 2 ? pS2 : pS3));
-    };
+    QG_LDS uint8_t* const pP0 = (QG_LDS uint8_t*)pn0;
+    QG_LDS uint8_t* const pP1 = (QG_LDS uint8_t*)pn1;
+    // stage and panel of K-tile S (mod 8), two-stage form
+    auto stage = [&](auto SC) __attribute__((always_inline)) { return (decltype(SC)::value & 1) ? pS1 : pS0; };
+    auto panel = [&](auto SC) __attribute__((always_inline)) { return (decltype(SC)::value & 4) ? pP1 : pP0; };
 
     auto rsrc = [&](const uint8_t* base, bool valid) __attribute__((always_inline)) {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, valid ? 0x7FFFFFFFu : 0u,
@@ -266,19 +300,56 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
         Src s;
         s.a = rsrc(A + (long long)kt * BKB, v);
         s.b = rsrc(B + (long long)kt * b_kstep, v);
-        s.sc = rsrc(sc_base + kt * sc_kstep, v);
+        // PANEL: the panel's first K-tile, counted from K = 0 (kt0 % 4 for slices that start inside a panel)
+        s.sc = rsrc(sc_base + (PANEL ? kt - ((kt0 + kt) & 3) : kt) * sc_kstep, v);
         return s;
     };
-    // DMA d (0 .. NDMA-1) of a K-tile into stage st: 0-3 A, 4-7 B, then scales
-    auto dma = [&](QG_LDS uint8_t* st, const Src& s, int d) __attribute__((always_inline)) {
+    // DMA d (0 .. ndma-1) of a K-tile into stage st: 0-3 A, 4-7 B, then scales
+    // (PANEL: of this and the next three K-tiles into panel pn)
+    auto dma = [&](QG_LDS uint8_t* st, QG_LDS uint8_t* pn, const Src& s, int d) __attribute__((always_inline)) {
         if (d < 4) dma16_buf(s.a, st + (4 * w + d) * 1024, aoff[d], 0);
         else if (d < 8) {
             if constexpr (NTB) dma16_buf_nt(s.b, st + OPB + (4 * w + d - 4) * 1024, boff[d - 4], 0);
             else dma16_buf(s.b, st + OPB + (4 * w + d - 4) * 1024, boff[d - 4], 0);
         }
-        else if (d == 8) dma4_buf(s.sc, st + sc_dst[0], sc_voff[0], 0);
-        else dma4_buf(s.sc, st + sc_dst[SCD - 1], sc_voff[SCD - 1], 0);
+        else if constexpr (PANEL) dma16_buf(s.sc, pn + sc_dst[d == 8 ? 0 : SCD - 1], sc_voff[d == 8 ? 0 : SCD - 1], 0);
+        else dma4_buf(s.sc, st + sc_dst[d == 8 ? 0 : SCD - 1], sc_voff[d == 8 ? 0 : SCD - 1], 0);
     };
+
+    // ---- SPEC: the DMA waves ----
+    // Keep the ring full: K-tile t + 4 goes into K-tile t's stage behind the
+    // barrier that frees it, the barrier itself waits for K-tile t + 1 (the
+    // K-tiles after it stay in flight: two, of at least NB DMAs each).
+    if constexpr (SPEC) {
+        if (tid >= 256) {
+            constexpr int NB = 8 + (PANEL ? 0 : SCD);
+            auto fill = [&](int t) __attribute__((always_inline)) {
+                const Src src = sources(t);
+                QG_LDS uint8_t* st = pS0 + (t & 3) * STAGE;
+                QG_LDS uint8_t* pn = pP0 + (PANEL ? (((kt0 + t) >> 2) & 1) * PAN : 0);
+                if (!PANEL || t == 0 || ((kt0 + t) & 3) == 0) {
+#pragma unroll
+                    for (int d = 8; d < 8 + SCD; ++d) dma(st, pn, src, d);
+                }
+#pragma unroll
+                for (int d = 0; d < 8; ++d) dma(st, pn, src, d);
+            };
+            auto landed = [&](int t) __attribute__((always_inline)) {    // K-tile t is in LDS
+                if (t + 2 < nk) wait_vmcnt<2 * NB>();
+                else if (t + 1 < nk) wait_vmcnt<NB>();
+                else wait_vmcnt<0>();
+                asm volatile("s_barrier" ::: "memory");
+            };
+            for (int t = 0; t < min(nk, 3); ++t) fill(t);
+            landed(0);
+            if (nk > 3) fill(3);
+            for (int t = 0; t < nk; ++t) {
+                landed(t + 1);
+                if (t + 4 < nk) fill(t + 4);
+            }
+            return;
+        }
+    }
 
     f32x4 acc[4][4];
 #pragma unroll
@@ -286,8 +357,10 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     i32x8 af[4], bf[2];
-    f32x4 part[2];
-    float fs[4];
+    int xa[4], xb[2];            // MX: E8M0 bytes of the lane's rows, beside af and bf
+    float fa[4], fb = 0.f;       // BSF32: the next K-tile's row scales and weight scale
+    f32x4 part[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    float fs[4] = {0.f, 0.f, 0.f, 0.f};
     // fragment chunks of row l16: fp8 q and q + 4; fp4 2q and 2q + 1 (the
     // two MFMAs of a 256-element K-tile, scale bytes 2q and 2q + 1)
     const int ca = FP4 ? 2 * q : q, cb = FP4 ? 2 * q + 1 : q + 4;
@@ -303,94 +376,160 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void mid_gemm_kernel(cons
         // zero scale operands select the unscaled fp8 MFMA (a plain product)
         return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, a, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
     };
-    auto rescale = [&](int i, int j, int x) __attribute__((always_inline)) {
+    auto rescale = [&](int i, int j, int x, float f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[x][e], fs[i], acc[i][j][e]);
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[x][e], f, acc[i][j][e]);
     };
 
-    // K-tile t (local index) from stage ST; the 9 DMAs of K-tile
-    // t + STAGES - 1 go into the stage K-tile t - 1 read (freed by this
-    // barrier), one after each of the first 9 MFMAs; the barrier waits for
-    // K-tile t's DMAs only (the later K-tiles' 9 (STAGES - 2) stay in flight)
-    auto ktile = [&](auto STC, int t) __attribute__((always_inline)) {
-        constexpr int ST = decltype(STC)::value;
-        QG_LDS uint8_t* cur = stage(mid::I<ST>{});
-        QG_LDS uint8_t* nxt = stage(mid::I<ST + STAGES - 1>{});
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NDMA * (STAGES - 2)) : "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        const QG_LDS uint8_t* sA = cur + wm * 64 * BKB;
-        const QG_LDS uint8_t* sB = cur + OPB + wn * 64 * BKB;
-        bf[0] = frag(sB, rdb0, rdb1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) af[i] = frag(sA + 16 * i * BKB, rd8, rd8b);
+    // A block i, or B block j into bf[j & 1], of the K-tile in stage st, with
+    // its rows' scales (PANEL: at pn): MX fp8 byte q, fp4 bytes 2q and
+    // 2q + 1; BSF32 the floats
+    auto read_a = [&](const QG_LDS uint8_t* st, const QG_LDS uint8_t* pn, int i) __attribute__((always_inline)) {
+        const int r = wm * 64 + 16 * i + l16;
+        af[i] = frag(st + (wm * 64 + 16 * i) * BKB, rd8, rd8b);
+        const QG_LDS uint8_t* pa = PANEL ? pn + r * PROW : st + SA_OFF + r * KTB;
+        if constexpr (!MX) fa[i] = *(const QG_LDS float*)pa;
+        else xa[i] = FP4 ? *(const QG_LDS uint16_t*)(pa + 2 * q) : pa[q];
+    };
+    auto read_b = [&](const QG_LDS uint8_t* st, const QG_LDS uint8_t* pn, int j) __attribute__((always_inline)) {
+        bf[j & 1] = frag(st + OPB + (wn * 64 + 16 * j) * BKB, rdb0, rdb1);
+        const QG_LDS uint8_t* sc = PANEL ? pn + 128 * PROW : st + SB_OFF;
         if constexpr (MX) {
-            // E8M0 bytes of the lane's rows: fp8 byte q, fp4 bytes 2q, 2q + 1
-            int sa[4], sb[4];
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const QG_LDS uint8_t* pa = cur + SA_OFF + (wm * 64 + 16 * x + l16) * KTB;
-                const QG_LDS uint8_t* pb = cur + SB_OFF + (wn * 64 + 16 * x + l16) * KTB;
-                sa[x] = FP4 ? *(const QG_LDS uint16_t*)(pa + 2 * q) : pa[q];
-                sb[x] = FP4 ? *(const QG_LDS uint16_t*)(pb + 2 * q) : pb[q];
-            }
-            const Src src = sources(t + STAGES - 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const int j = k >> 2, i = k & 3;
-                if (i == 0 && j < 3) bf[(j + 1) & 1] = frag(sB + (j + 1) * 16 * BKB, rdb0, rdb1);
-                const i32x8& b = bf[j & 1];
-                if constexpr (FP4) {
-                    const i32x8 b0 = i32x8{b[0], b[1], b[2], b[3], 0, 0, 0, 0};
-                    const i32x8 b1 = i32x8{b[4], b[5], b[6], b[7], 0, 0, 0, 0};
-                    const i32x8 a0 = i32x8{af[i][0], af[i][1], af[i][2], af[i][3], 0, 0, 0, 0};
-                    const i32x8 a1 = i32x8{af[i][4], af[i][5], af[i][6], af[i][7], 0, 0, 0, 0};
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b0, a0, acc[i][j], kFmtFp4, kFmtFp4,
-                                                                                 0, sb[j], 0, sa[i]);
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b1, a1, acc[i][j], kFmtFp4, kFmtFp4,
-                                                                                 1, sb[j], 1, sa[i]);
-                } else {
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, af[i], acc[i][j], kFmtFp8,
-                                                                                 kFmtFp8, 0, sb[j], 0, sa[i]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                if (k < NDMA) dma(nxt, src, k);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            const float sb = *(const QG_LDS float*)(cur + SB_OFF);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                fs[i] = *(const QG_LDS float*)(cur + SA_OFF + 4 * (wm * 64 + 16 * i + l16)) * sb;
-            const Src src = sources(t + STAGES - 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const int j = k >> 2, i = k & 3;
-                if (i == 0 && j < 3) bf[(j + 1) & 1] = frag(sB + (j + 1) * 16 * BKB, rdb0, rdb1);
-                part[k & 1] = mfma_part(bf[j & 1], af[i]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (k > 0) rescale((k - 1) & 3, (k - 1) >> 2, (k - 1) & 1);
-                if (k < NDMA) dma(nxt, src, k);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            rescale(3, 3, 1);
+            const QG_LDS uint8_t* pb = sc + (wn * 64 + 16 * j + l16) * (PANEL ? PROW : KTB);
+            xb[j & 1] = FP4 ? *(const QG_LDS uint16_t*)(pb + 2 * q) : pb[q];
+        } else if (j == 0) {
+            fb = *(const QG_LDS float*)sc;
         }
     };
-
-    // ---- prologue: K-tiles 0 .. STAGES - 2 into their stages ----
-    mid::static_for<STAGES - 1>([&](auto SC) __attribute__((always_inline)) {
-        const Src s0 = sources(decltype(SC)::value);
+    // MFMA k of the K-tile (block row k & 3, block column k >> 2) and, fp32
+    // scales, the rescale of the one before (`last`: the scale of the K-tile
+    // before's block 15)
+    auto product = [&](int k, float last) __attribute__((always_inline)) {
+        const int j = k >> 2, i = k & 3;
+        const i32x8 &b = bf[j & 1], &a = af[i];
+        if constexpr (!MX) {
+            part[k & 1] = mfma_part(b, a);
+        } else if constexpr (FP4) {
+            const i32x8 b0 = i32x8{b[0], b[1], b[2], b[3], 0, 0, 0, 0};
+            const i32x8 b1 = i32x8{b[4], b[5], b[6], b[7], 0, 0, 0, 0};
+            const i32x8 a0 = i32x8{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
+            const i32x8 a1 = i32x8{a[4], a[5], a[6], a[7], 0, 0, 0, 0};
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b0, a0, acc[i][j], kFmtFp4, kFmtFp4, 0,
+                                                                         xb[j & 1], 0, xa[i]);
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b1, a1, acc[i][j], kFmtFp4, kFmtFp4, 1,
+                                                                         xb[j & 1], 1, xa[i]);
+        } else {
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, a, acc[i][j], kFmtFp8, kFmtFp8, 0,
+                                                                         xb[j & 1], 0, xa[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!MX) {
+            if (k == 0) rescale(3, 3, 1, last);
+            else rescale((k - 1) & 3, (k - 1) >> 2, (k - 1) & 1, fs[(k - 1) & 3]);
+        }
+    };
+    auto scales = [&]() __attribute__((always_inline)) {
+        const float last = fs[3];
+        if constexpr (!MX) {
 #pragma unroll
-        for (int d = 0; d < NDMA; ++d) dma(stage(SC), s0, d);
-    });
-    int t = 0;
-    for (; t + STAGES <= nk; t += STAGES)
-        mid::static_for<STAGES>([&](auto SC) __attribute__((always_inline)) { ktile(SC, t + decltype(SC)::value); });
-    mid::static_for<STAGES - 1>([&](auto SC) __attribute__((always_inline)) {
-        if (t + decltype(SC)::value < nk) ktile(SC, t + decltype(SC)::value);
-    });
-    wait_vmcnt<0>();    // the DMAs past the slice still write zeros
+            for (int i = 0; i < 4; ++i) fs[i] = fa[i] * fb;
+        }
+        return last;
+    };
+
+    // A K-tile is 16 MFMAs in four column blocks j, block j + 1's operands
+    // read under block j's MFMAs.  A and block 0 are in registers from the
+    // K-tile before: the barrier stands before block 3, when every wave has
+    // read all of K-tile t, so that K-tile t + 1's first operands -- A block
+    // by block behind its last MFMA -- are read under block 3.  (With the
+    // barrier at the K-tile's start a wave, alone on its SIMD with four
+    // stages, waited for LDS once per K-tile with nothing to run.)
+    if constexpr (SPEC) {
+        asm volatile("s_barrier" ::: "memory");     // K-tile 0 has landed
+        auto scales_of = [&](int t) __attribute__((always_inline)) {
+            const int x = kt0 + t;
+            return pP0 + (PANEL ? ((x >> 2) & 1) * PAN + (x & 3) * KTB : 0);
+        };
+        read_b(pS0, scales_of(0), 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) read_a(pS0, scales_of(0), i);
+        for (int t = 0; t < nk; ++t) {
+            const QG_LDS uint8_t *cur = pS0 + (t & 3) * STAGE, *nxt = pS0 + ((t + 1) & 3) * STAGE;
+            const QG_LDS uint8_t *pc = scales_of(t), *pn = scales_of(t + 1);
+            const float last = scales();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int j = k >> 2, i = k & 3;
+                if (k == 12) {
+                    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_b(nxt, pn, 0);
+                } else if (i == 0) {
+                    read_b(cur, pc, j + 1);
+                }
+                product(k, last);
+                if (k >= 12) read_a(nxt, pn, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    } else {
+        // K-tile t (local index, t % 8 = S).  The barrier also waits for
+        // K-tile t + 1's DMAs; those of K-tile t + 2 into the freed stage
+        // follow it, four under block 3 and the rest under the next
+        // K-tile's blocks 0-2.
+        auto ktile = [&](auto SC, int t) __attribute__((always_inline)) {
+            constexpr int S = decltype(SC)::value;
+            using Nxt = mid::I<(S + 1) & 7>;                        // K-tile t + 1; t - 1's stage is the same
+            constexpr int ND = ndma(S + 1);
+            const QG_LDS uint8_t *pc = panel(SC) + (S & 3) * KTB, *pn = panel(Nxt{}) + ((S + 1) & 3) * KTB;
+            const float last = scales();
+            const Src sp = sources(t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int j = k >> 2, i = k & 3;
+                if (k == 12) {
+                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_b(stage(Nxt{}), pn, 0);
+                } else if (i == 0) {
+                    read_b(stage(SC), pc, j + 1);
+                }
+                product(k, last);
+                if (k + 4 < ND) {
+                    dma(stage(Nxt{}), panel(Nxt{}), sp, k + 4);
+                } else if (k >= 12) {
+                    dma(stage(SC), panel(mid::I<(S + 2) & 7>{}), sources(t + 2), k - 12);
+                    read_a(stage(Nxt{}), pn, i);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // prologue: K-tile 0 and the first four DMAs of K-tile 1 into their
+        // stages, K-tile 0's first operands into registers
+        {
+            const Src s0 = sources(0), s1 = sources(1);
+#pragma unroll
+            for (int d = 0; d < ndma(0); ++d) dma(pS0, pP0, s0, d);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) dma(pS1, pP0, s1, d);
+            asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            read_b(pS0, pP0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) read_a(pS0, pP0, i);
+        }
+        constexpr int UN = PANEL ? 8 : 2;
+        int t = 0;
+        for (; t + UN <= nk; t += UN)
+            mid::static_for<UN>([&](auto SC) __attribute__((always_inline)) { ktile(SC, t + decltype(SC)::value); });
+        mid::static_for<UN - 1>([&](auto SC) __attribute__((always_inline)) {
+            if (t + decltype(SC)::value < nk) ktile(SC, t + decltype(SC)::value);
+        });
+        wait_vmcnt<0>();    // the DMAs past the slice still write zeros
+    }
+    if constexpr (!MX) rescale(3, 3, 1, fs[3]);
 
     // ---- output: lane holds C[16i + l16][16j + 4q + 0..3] of the wave's block ----
     const int mw = m0 + wm * 64 + l16, nw0 = n0 + wn * 64 + 4 * q;
