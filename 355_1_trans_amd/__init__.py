@@ -32,6 +32,8 @@ buffer per (device, stream); pass a tensor to supply your own, or
 ``workspace=False`` to run without split-K.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 from functools import lru_cache
 from pathlib import Path
 
@@ -170,6 +172,47 @@ def lib():
     return L
 
 
+# The library functions _fast.so calls, in its order (csrc/host/fast.cpp, struct Lib).
+_FAST_CALLS = (
+    "qgemm_quant_fp8_blockscale_act", "qgemm_quant_fp8_e8m0_act", "qgemm_quant_mxfp8", "qgemm_quant_mxfp4",
+    "qgemm_e8m0_shuffle_bytes", "gemm_a8w8_blockscale_bpreshuffle", "gemm_a8w8_blockscale_bpreshuffle_workspace_bytes",
+    "gemm_a8w8_blockscale_ldsbypass", "gemm_a8w8_blockscale_ldsbypass_workspace_bytes", "qgemm_ldsbypass_b_bytes",
+    "gemm_a8w8_mxfp8", "gemm_a8w8_mxfp8_workspace_bytes", "gemm_a4w4_mxfp4", "gemm_a4w4_mxfp4_workspace_bytes",
+    "gemm_a4w4_mxfp4_bpreshuffle_kid", "gemm_a4w4_mxfp4_bpreshuffle_kid_workspace_bytes",
+    "launch_blockscale_bpreshuffle")
+
+
+class _NoFast:
+    """Without _fast.so every call takes the wrappers' own Python code."""
+
+    @staticmethod
+    def gemm(*_):
+        return None
+
+    @staticmethod
+    def quant(*_):
+        return None
+
+
+def fast():
+    """The native form of the wrappers' plain calls (_fast.so, built with the
+    library): ``gemm`` and ``quant`` return None for a call that the Python
+    code has to check or make."""
+    return _fast_module() if LIB_PATH.exists() else _NoFast
+
+
+@lru_cache(None)
+def _fast_module():
+    path = _PKG / "_fast.so"
+    if not path.exists():
+        return _NoFast
+    loader = importlib.machinery.ExtensionFileLoader("_fast", str(path))
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_fast", path, loader=loader))
+    loader.exec_module(mod)
+    mod.bind(*[ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _FAST_CALLS])
+    return mod
+
+
 def last_launch():
     """Kernel instantiations launched by this thread's most recent library
     call (qgemm_last_launch), e.g. 'wide_gemm<fp8,MX,RAW,bf16,pb16>'."""
@@ -253,6 +296,10 @@ def _out_code(dtype):
 
 def gemm_a8w8_mxfp8(A, B, A_scale, B_scale, dtype=torch.bfloat16, out=None, workspace=None):
     """MXFP8 TN GEMM: A [M,K] e4m3, B [N,K] e4m3, A_scale [M,K/32], B_scale [N,K/32] E8M0 bytes."""
+    if out is None and workspace is None:
+        y = fast().gemm(2, A, B, A_scale, B_scale, dtype, 0, _WORKSPACES)
+        if y is not None:
+            return y
     dev = _require_gpu(A, B, A_scale, B_scale)
     m, k = A.shape
     n = B.shape[0]
@@ -278,6 +325,10 @@ def gemm_a8w8_mxfp8(A, B, A_scale, B_scale, dtype=torch.bfloat16, out=None, work
 
 def gemm_a4w4_mxfp4(A, B, A_scale, B_scale, dtype=torch.bfloat16, out=None, workspace=None):
     """MXFP4 A4W4 GEMM: A [M,K/2], B [N,K/2] packed e2m1 bytes, scales [rows,K/32] E8M0."""
+    if out is None and workspace is None:
+        y = fast().gemm(3, A, B, A_scale, B_scale, dtype, 0, _WORKSPACES)
+        if y is not None:
+            return y
     dev = _require_gpu(A, B, A_scale, B_scale)
     m, kb = A.shape
     n = B.shape[0]
@@ -334,6 +385,10 @@ def gemm_a4w4(A, B, A_scale, B_scale, out=None, bias=None, alpha=1.0, beta=0.0, 
         raise NotImplementedError("gemm_a4w4: bias, alpha and beta are not supported")
     if not bpreshuffle:
         raise NotImplementedError("gemm_a4w4: row-major B goes through gemm_a4w4_mxfp4")
+    if out is None and workspace is None and grid_blocks == 0 and kernel_id == 0:
+        y = fast().gemm(4, A, B, A_scale, B_scale, torch.bfloat16 if dtype is None else dtype, 0, _WORKSPACES)
+        if y is not None:
+            return y
     dev = _require_gpu(A, B, A_scale, B_scale)
     if dtype is None:
         dtype = out.dtype if out is not None else torch.bfloat16
@@ -369,6 +424,10 @@ def gemm_a8w8_bpreshuffle(A, B_kpanel, A_scale, B_scale, dtype=torch.bfloat16, o
     A_scale fp32 [M,K/128] (row-major, BASELINE) or a [M,K/128] view with
     strides (1, M) (the reference's column-major [K/128][M]); B_scale fp32
     [ceil(N/128), K/128]."""
+    if out is None and workspace is None:
+        y = fast().gemm(0, A, B_kpanel, A_scale, B_scale, dtype, 0, _WORKSPACES)
+        if y is not None:
+            return y
     dev = _require_gpu(A, B_kpanel, A_scale, B_scale)
     m, k = A.shape
     if B_kpanel.dim() != 3 or B_kpanel.shape[0] * 128 != k or B_kpanel.shape[2] != 128:
@@ -448,6 +507,10 @@ def ldsbypass_repack(B_kpanel, out=None):
 def gemm_a8w8_ldsbypass(A, B_pp, A_scale, B_scale, n, dtype=torch.bfloat16, out=None, workspace=None):
     """Block-scale FP8 (fp32 scales) with B given as B'' (``ldsbypass_repack``
     or ``ldsbypass_pack_b``); A, A_scale, B_scale as in gemm_a8w8_bpreshuffle."""
+    if out is None and workspace is None:
+        y = fast().gemm(1, A, B_pp, A_scale, B_scale, dtype, n, _WORKSPACES)
+        if y is not None:
+            return y
     dev = _require_gpu(A, B_pp, A_scale, B_scale)
     m, k = A.shape
     kg = k // 128

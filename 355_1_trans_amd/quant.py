@@ -24,7 +24,7 @@ import ctypes
 
 import torch
 
-from . import _check, _record, _require_gpu, _stream, lib
+from . import _check, _record, _require_gpu, _stream, fast, lib
 
 IN_FP32, IN_BF16 = 0, 1
 
@@ -52,6 +52,10 @@ def quant_fp8_blockscale(x, block="1x128", scale_layout="mk"):
     (scale_layout "mk": row-major; "km": the BPS column-major [K/128][M],
     returned as the [M, K/128] view with strides (1, M)); block "128x128"
     gives scale [ceil(N/128), K/128]."""
+    if block == "1x128" and scale_layout in ("mk", "km"):
+        qs = fast().quant(0 if scale_layout == "mk" else 1, x)
+        if qs is not None:
+            return qs
     code, ld = _source(x, 128)
     rows, k = x.shape
     kg = k // 128
@@ -81,6 +85,10 @@ def quant_fp8_e8m0_blockscale(x, block="1x128"):
     view with strides (1, M) of column-major bytes, as
     blockscale_bpreshuffle.gemm_a8w8_blockscale_bpreshuffle takes it;
     "128x128": e [N/128, K/128] (N % 128 == 0 for that kernel)."""
+    if block == "1x128":
+        qe = fast().quant(2, x)
+        if qe is not None:
+            return qe
     code, ld = _source(x, 128)
     rows, k = x.shape
     kg = k // 128
@@ -118,13 +126,17 @@ def _quant_mx(x, fp4, shuffle):
 
 def quant_mxfp8(x, shuffle=False):
     """(q float8_e4m3fn [rows, K], e uint8 [rows, K/32] or the e8m0_shuffle bytes)."""
+    qe = fast().quant(4 if shuffle else 3, x)
+    if qe is not None:
+        return qe
     q, e = _quant_mx(x, False, shuffle)
     return q.view(torch.float8_e4m3fn), e
 
 
 def quant_mxfp4(x, shuffle=False):
     """(q uint8 [rows, K/2] packed e2m1, e uint8 [rows, K/32] or the e8m0_shuffle bytes)."""
-    return _quant_mx(x, True, shuffle)
+    qe = fast().quant(6 if shuffle else 5, x)
+    return _quant_mx(x, True, shuffle) if qe is None else qe
 
 
 def e8m0_shuffle(e):
