@@ -21,6 +21,7 @@
 #include "burst_gemm.hpp"
 #include "decode_gemm.hpp"
 #include "mid_gemm.hpp"
+#include "ring_gemm.hpp"
 #include "runs_gemm.hpp"
 #include "slice_gemm.hpp"
 #include "stream_gemm.hpp"
@@ -537,6 +538,83 @@ TailPlan plan_tail(int m, int n, int k_tiles, int batch, int cus) {
     return tp;
 }
 
+// Ring kernel (ring_gemm.hpp): M <= 64, 16 mb rows and 16 nb columns per
+// workgroup, K slices of whole stages (4 K-tiles).  (nb, split) is the pair
+// with the least modelled time: a fixed part, the extra launch and the
+// partials of a split, and per stage and round the operands' rows, B's share
+// dearer the more CUs stream at once (us, least squares over 560 graph-
+// replayed (shape, nb, split) triples, M = 1-64, N = 1536-24576, K = 1536-16384;
+// the pick is within 0.6% of the best pair in the geometric mean).  `rows`:
+// row-major MX operands, whose 16 / 32-byte scale pieces cost their own DMAs.
+constexpr int kRingMaxSplit = 8;
+struct RingPlan {
+    bool ok = false;
+    int mb = 1, nb = 1, splitk = 1, st_per_split = 1, n_tiles = 1;
+    size_t ws_bytes = 0;
+};
+RingPlan plan_ring(int m, int n, int kt, int batch, bool rows, bool fp4, int cus, bool split) {
+    RingPlan r;
+    if (m < 1 || m > 64 || n < 1 || kt < 1 || batch < 1) return r;
+    r.mb = m <= 16 ? 1 : m <= 32 ? 2 : 4;
+    const int nst = ceil_div(kt, 4);
+    const double planes_mb = 4e-6 * m * n * batch;
+    if ((long long)m * n >= (1LL << 29)) split = false;
+    double best = 0;
+    for (int nb = 1; nb <= (r.mb == 4 ? 2 : 4); nb *= 2) {
+        const long long tiles = (long long)ceil_div(n, 16 * nb) * batch;
+        for (int sp = 1; sp <= (split ? kRingMaxSplit : 1); ++sp) {
+            const int sps = ceil_div(nst, sp);
+            if (sp > 1 && (sps < 2 || ceil_div(nst, sps) != sp)) continue;
+            const long long wgs = tiles * sp, rounds = (wgs + cus - 1) / cus;
+            const double conc = (double)std::min<long long>(wgs, cus) / cus;
+            const double stage = -0.0425 + 0.133 * r.mb + nb * (0.140 + 0.150 * conc) +
+                                 (rows ? (fp4 ? 0.017 : 0.0085) * (r.mb + nb) : 0.0);
+            const double us = 3.8 + (sp > 1 ? 1.87 + 0.86 * sp * planes_mb : 0.0) + stage * sps * rounds +
+                              1.1 * (rounds - 1);
+            if (r.ok && us >= best) continue;
+            best = us;
+            r.ok = true;
+            r.nb = nb;
+            r.splitk = sp;
+            r.st_per_split = sps;
+            r.n_tiles = ceil_div(n, 16 * nb);
+        }
+    }
+    r.ws_bytes = r.splitk > 1 ? kCounterBytes + (size_t)r.splitk * batch * m * n * 4 : 0;
+    return r;
+}
+// an AUTO call takes its ring plan when its split's planes fit the workspace
+// at hand (none: only unsplit plans); what fitted without it still runs
+bool ring_fits(const RingPlan& p, bool have_ws, size_t ws_cap) {
+    return p.ok && (p.splitk == 1 || (have_ws && p.ws_bytes <= ws_cap));
+}
+// the ring kernel's arguments but for the load ranges
+qg::RingArgs ring_args(const RingPlan& p, const TileArgs& t, bool bf16, void* ws) {
+    qg::RingArgs a{};
+    a.t = t;
+    a.splitk = p.splitk;
+    a.st_per_split = p.st_per_split;
+    a.n_tiles = p.n_tiles;
+    a.bf16 = bf16;
+    if (p.splitk > 1) a.ws = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kCounterBytes);
+    return a;
+}
+// sums a split's partial planes into C
+hipError_t ring_reduce(const qg::RingArgs& a, int batch, bool bf16, hipStream_t stream) {
+    if (a.splitk == 1) return hipSuccess;
+    qg::SplitReduceArgs r{};
+    r.ws = a.ws;
+    r.c = a.t.c;
+    r.m = a.t.m;
+    r.n = a.t.n;
+    r.ldc = a.t.ldc;
+    r.c_vec = a.t.c_vec;
+    r.splitk = a.splitk;
+    r.batch = batch;
+    r.c_batch = a.t.c_batch;
+    return qg::launch_splitk_reduce(r, bf16, stream);
+}
+
 // Kernel routes of the fp32 block-scale entries (QGEMM_KID_* in qgemm.h):
 // AUTO resolves to one of the others by the plans above; a forced route
 // runs that kernel with its own plan (tile shape and K split), or fails
@@ -549,16 +627,58 @@ struct BsfRoute {
     qg::BurstPlan bp;
     Plan pl;
     TailPlan tp;
+    RingPlan rg;
     size_t ws_bytes = 0;
 };
 
-BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bool frag, int kid, bool have_ws) {
+// AUTO's rule for the ring kernel on fp32 block scales (batch 1), from sweeps
+// of both layouts over M = 1-64, N = 256-24576, K = 1536-16384 (graph-replayed
+// over rotating weights; factors: the route below / the ring):
+//  * M <= 16, where the burst kernel's unstaged loads win at most N (ring
+//    0.82-1.0): only narrow N with long K, which no other plan splits as
+//    evenly (N <= 768, K >= 7168 1.08-1.38, M <= 4 from 12288 on, before 0.91-0.99;
+//    N <= 2112, K = 16384 1.03-1.27);
+//  * M = 17-32: narrow N (N <= 768: K = 4096 1.16-1.67, 7168 1.15-1.36; 16384
+//    1.05-1.4 up to 2112), 2112 - 7168 with K >= 7168 (1.04-1.7; K-panel B
+//    past N = 4096 only to K = 8192, at 12288 0.89), N to 8192 at K = 4096
+//    (1.03-1.07), N = 12288 - 16384 at K <= 2048 (1.04-1.10; K = 16384
+//    0.84-1.0);
+//  * M = 33-64: N <= 4096 (1.04-1.87) and to 8192 at K = 2560 - 6144 (1.14-2.4;
+//    7168 at N <= 7168 1.05-1.14; wider or longer loses, 0.7-1.0).  N = 1025 -
+//    1536 near K = 7168 and N <= 768 near K = 8192 with M <= 32 stay on the
+//    burst kernel, N = 7168 at K <= 2048 too (ring 1.02-1.11 on these).
+bool ring_bsf32(int m, int n, int kt, int batch, bool frag) {
+    if (batch != 1 || n < 256 || m > 64) return false;
+    const bool long_k = kt >= 96;
+    if (m <= 16) return n <= 768 ? kt >= (m <= 4 ? 96 : 56) : n <= 2560 && long_k;
+    if (m <= 32) {
+        if (n <= 768) return long_k || (kt >= 32 && kt < 64);
+        if (n <= 2048) return long_k;
+        if (n <= 4096) return kt >= 56;
+        if (n <= 8192) return (kt >= 24 && kt <= 48) || (n <= 7168 && kt >= 56 && (frag || kt <= 64));
+        return n >= 12288 && n <= 16384 && kt >= 12 && kt <= 16;
+    }
+    if (n <= 4096) return kt >= 12 && !(n > 1024 && n <= 1536 && kt > 48 && kt < 64);
+    return n <= 8192 && kt > 16 && kt <= (n <= 7168 ? 56 : 48);
+}
+
+BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bool frag, int kid, bool have_ws,
+                     size_t ws_cap) {
     BsfRoute r;
     r.kid = kid;
     if (m <= 0 || n <= 0 || k_tiles <= 0 || batch <= 0) return r;
     const int cus = device_cus();
     switch (kid) {
         case QGEMM_KID_AUTO: {
+            if (ring_bsf32(m, n, k_tiles, batch, frag)) {
+                r.rg = plan_ring(m, n, k_tiles, batch, false, false, cus, true);
+                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                    r.kid = QGEMM_KID_RING;
+                    r.ws_bytes = r.rg.ws_bytes;
+                    r.ok = true;
+                    return r;
+                }
+            }
             r.bp = plan_bsf32_burst(m, n, k_tiles, batch);
             if (r.bp.ok) {
                 r.ws_bytes = burst_ws_bytes(r.bp, m, n, batch);
@@ -598,6 +718,12 @@ BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bo
             r.ws_bytes = burst_ws_bytes(r.bp, m, n, batch);
             if (r.bp.splitk > 1 && !have_ws) r.bp = qg::burst_plan(m, n, k_tiles, batch, cus, kMaxCounters, false, 1);
             r.ok = r.bp.ok;
+            return r;
+        case QGEMM_KID_RING:
+            r.rg = plan_ring(m, n, k_tiles, batch, false, false, cus, true);
+            r.ws_bytes = r.rg.ws_bytes;
+            if (r.rg.splitk > 1 && !have_ws) r.rg = plan_ring(m, n, k_tiles, batch, false, false, cus, false);
+            r.ok = r.rg.ok;
             return r;
         default:
             return r;
@@ -1036,6 +1162,18 @@ hipError_t run_bsf32(const BsfRoute& r, const TileArgs& t, int batch, bool frag,
     switch (r.kid) {
         case QGEMM_KID_BURST:
             return run_burst(t, batch, r.bp, frag, b_bytes, bf16, ws, stream);
+        case QGEMM_KID_RING: {
+            qg::RingArgs a = ring_args(r.rg, t, bf16, ws);
+            a.a_bytes = (long long)(t.m - 1) * t.lda + t.kbytes;
+            a.b_bytes = b_bytes;
+            a.sfa_bytes = 4 * ((long long)(t.m - 1) * t.sfa_sm + (long long)(k_tiles - 1) * t.sfa_sk + 1);
+            a.sfb_bytes = 4 * ((long long)((t.n - 1) / 128) * t.sfb_sn + k_tiles);
+            // A's scales in panels: whole stages, K-contiguous rows of 16-byte units
+            const bool panel = k_tiles % 4 == 0 && t.sfa_sk == 1 && t.sfa_sm % 4 == 0 && aligned(t.sfa, 16) &&
+                               (batch == 1 || t.sfa_batch % 4 == 0);
+            const hipError_t st = qg::launch_ring_bs(a, frag, r.rg.mb, r.rg.nb, panel, batch, stream);
+            return st != hipSuccess ? st : ring_reduce(a, batch, bf16, stream);
+        }
         case QGEMM_KID_MID:
             return run_mid(t, batch, r.pl, bf16, frag ? qg::MidKind::BS_FRAG : qg::MidKind::BS_KPANEL, ws, ws_bytes,
                            k_tiles, stream);
@@ -1137,6 +1275,7 @@ struct MxRoute {
     qg::BurstPlan bp;
     BandPlan bd;
     RunsPlan rn;
+    RingPlan rg;
     int wsplit = 1;    // K slices of the four-wave kernel (plan_wide_split)
     size_t ws_bytes = 0;
 };
@@ -1205,6 +1344,42 @@ qg::BurstPlan plan_mx_burst(int m, int n, int k_tiles, int batch, bool gate) {
     return qg::burst_plan(m, n, k_tiles, batch, device_cus(), kMaxCounters, gate, 16, true);
 }
 
+// The ring kernel's loads: 16-byte units of A and B rows, scale rows by
+// dwords; in panels where whole stages of scales start on 16 bytes.
+bool ring_ok(const opus_gemm_scale_kargs& a) { return band_ok(a); }
+bool ring_panels(const opus_gemm_scale_kargs& a, bool fp4) {
+    return runs_ok(a) && a.k / (fp4 ? 256 : 128) % 4 == 0;
+}
+// AUTO's rule for it (batch 1, scale panels), from sweeps of both formats over
+// M = 1-64, N = 256-24576, K = 1536-16384 (graph-replayed over rotating
+// weights; factors: the route below / the ring; `row`: bytes of a row of B):
+//  * M <= 8: short K, where the row-streaming kernel is all latency (N <=
+//    12288: fp8 K <= 2048 1.15-1.7, 4096 with M > 4 1.01-1.38; fp4 K <= 7168
+//    1.02-1.6; at K = 16384 it reads 512-byte runs better, ring 0.74-1.05);
+//  * M = 9-16: a full round of 64-column tiles from 2 KB rows on (1.04-1.35;
+//    at N <= 8192 the burst and slice kernels win, ring 0.86-1.04), and narrow
+//    N with long K (1.0-1.34);
+//  * M = 17-32: the full round (1.17-1.49; rows of 3.5-4 KB keep the slice
+//    kernel, ring 0.95-1.04), narrow N with long K (1.1-1.4), N = 4097 - 8192
+//    with 2-4 KB rows (1.01-1.33, where the burst plans run in two waves);
+//  * M = 33-64, N <= 8192 (1.06-1.85): A's rows come once per 16-32 columns
+//    from LDS.  Wider N: the 128 x 128 kernel, which reads A once per 128.
+//    64 - 71 K-tiles with M > 40 stay on the row-run kernel at N <= 4096 and,
+//    MXFP4, on the slice kernel past N = 6144 (ring 1.15-1.34 there).
+bool ring_mx(int m, int n, int kt, bool fp4) {
+    const int row = kt * 128;
+    if (m > 64 || n < 256) return false;
+    if (m <= 8) return n <= 12288 && kt >= 8 && kt <= (fp4 ? (m > 4 ? 32 : 28) : m > 4 ? 32 : 16);
+    const bool round64 = n >= 12288 && n <= 16384;
+    if (m <= 16)
+        return (round64 && row >= 2048) || (n <= 2560 && kt * (fp4 ? 256 : 128) > 12288) || (n <= 768 && row >= 7168);
+    if (m <= 32) {
+        if (round64) return row >= 1024 && (row < 3584 || row > 4096);
+        return (n <= 2560 && row >= (n <= 768 ? 3072 : 7168)) || (n > 4096 && n <= 8192 && row >= 2048 && row <= 4096);
+    }
+    return n <= 8192 && row >= 1536 && !(m > 40 && kt >= 64 && kt < 72 && (n <= 4096 || (fp4 && n > 6144)));
+}
+
 MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws, size_t ws_cap) {
     MxRoute r;
     r.kid = kid;
@@ -1214,6 +1389,15 @@ MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws
     const int cus = device_cus();
     switch (kid) {
         case QGEMM_KID_AUTO: {
+            if (a.batch == 1 && ring_mx(a.m, a.n, kt, fp4) && ring_panels(a, fp4)) {
+                r.rg = plan_ring(a.m, a.n, kt, 1, true, fp4, cus, true);
+                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                    r.kid = QGEMM_KID_RING;
+                    r.ws_bytes = r.rg.ws_bytes;
+                    r.ok = true;
+                    return r;
+                }
+            }
             r.pl = plan_mx(a.m, a.n, kt, a.batch, bb, fp4);
             r.sp = plan_stream(a.m, a.n, a.k, a.batch, fp4);
             r.bp = plan_mx_burst(a.m, a.n, kt, a.batch, true);
@@ -1389,6 +1573,13 @@ MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws
             if (!r.rn.ok) return r;
             r.ws_bytes = r.rn.ws_bytes;
             break;
+        case QGEMM_KID_RING:
+            if (!ring_ok(a)) return r;
+            r.rg = plan_ring(a.m, a.n, kt, a.batch, true, fp4, cus, true);
+            r.ws_bytes = r.rg.ws_bytes;
+            if (r.rg.splitk > 1 && !have_ws) r.rg = plan_ring(a.m, a.n, kt, a.batch, true, fp4, cus, false);
+            if (!r.rg.ok) return r;
+            break;
         default:
             return r;
     }
@@ -1435,6 +1626,15 @@ hipError_t run_mx(const MxRoute& r, TileArgs t, const opus_gemm_scale_kargs& a, 
             }
             return r.kid == QGEMM_KID_SLICE ? qg::launch_slice(x, fp4, r.rn.mb, a.batch, bf16, stream)
                                             : qg::launch_runs(x, fp4, r.rn.mb, a.batch, bf16, stream);
+        }
+        case QGEMM_KID_RING: {
+            qg::RingArgs x = ring_args(r.rg, t, bf16, ws);
+            x.a_bytes = (long long)(a.m - 1) * a.stride_a + t.kbytes;
+            x.b_bytes = (long long)(a.n - 1) * a.stride_b + t.kbytes;
+            x.sfa_bytes = (long long)(a.m - 1) * a.stride_sfa + a.k / 32;
+            x.sfb_bytes = (long long)(a.n - 1) * a.stride_sfb + a.k / 32;
+            const hipError_t st = qg::launch_ring_mx(x, fp4, r.rg.mb, r.rg.nb, ring_panels(a, fp4), a.batch, stream);
+            return st != hipSuccess ? st : ring_reduce(x, a.batch, bf16, stream);
         }
         case QGEMM_KID_SKINNY:
         case QGEMM_KID_DECODE:
@@ -1676,6 +1876,7 @@ struct Mx4sRoute {
     bool ok = false;
     qg::BurstPlan bp;
     RunsPlan sl;       // SLICE
+    RingPlan rg;
     int qsplit = 1;    // QUAD: K slices (batch 1), fp32 partial planes + splitk_reduce
     size_t ws_bytes = 0;
 };
@@ -1698,7 +1899,17 @@ int plan_quad_split(const opus_gemm_mxfp4_scale_kargs& x, int cus) {
     while (s > 1 && kt % s) --s;
     return std::max(s, 1);
 }
-Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws) {
+// AUTO's rule for the ring kernel (batch 1; graph-replayed, the route below /
+// the ring): M = 33-64 from 24 K-tiles on (N = 2048 - 7168: 1.02-1.42; short
+// K 0.83-1.0), and one round of 64-column tiles at K >= 16384 from M = 17 on
+// (N = 13312 / 16384: 1.36-1.66).  At M <= 32 the burst kernel's 1 KB loads of
+// W16 blocks need no staging (ring 0.74-1.0); N <= 1536 stays on it too (1.0-1.16).
+bool ring_mx4s(int m, int n, int kt) {
+    if (n > 12288 && n <= 16384 && kt >= 64) return m > 16 && m <= 64;
+    return m > 32 && m <= 64 && n > 1536 && n <= 7168 && kt >= 24;
+}
+
+Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws, size_t ws_cap) {
     Mx4sRoute r;
     const int kt = x.k / 256;
     const int cus = device_cus();
@@ -1711,6 +1922,14 @@ Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws
     switch (kid) {
         case QGEMM_KID_AUTO: {
             r.ok = true;
+            if (x.grid_blocks == 0 && x.batch == 1 && ring_mx4s(x.m, x.n, kt)) {
+                r.rg = plan_ring(x.m, x.n, kt, 1, false, true, cus, true);
+                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                    r.kid = QGEMM_KID_RING;
+                    r.ws_bytes = r.rg.ws_bytes;
+                    return r;
+                }
+            }
             const bool quad_short = 2LL * ceil_div(x.n, 256) * x.batch >= cus && kt <= 4;
             if (x.grid_blocks == 0 && x.m > 8 && x.m <= 64) {
                 // the slice kernel on the row-major route's rule (one round of
@@ -1759,6 +1978,13 @@ Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws
             r.sl = plan_slice(x.m, x.n, kt, x.batch, have_ws);
             r.ok = x.grid_blocks == 0 && r.sl.ok;
             r.ws_bytes = r.sl.ws_bytes;
+            return r;
+        case QGEMM_KID_RING:
+            r.kid = kid;
+            r.rg = plan_ring(x.m, x.n, kt, x.batch, false, true, cus, true);
+            r.ws_bytes = r.rg.ws_bytes;
+            if (r.rg.splitk > 1 && !have_ws) r.rg = plan_ring(x.m, x.n, kt, x.batch, false, true, cus, false);
+            r.ok = x.grid_blocks == 0 && r.rg.ok;
             return r;
         default:
             return r;
@@ -1816,7 +2042,7 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
     hipError_t st = validate_mx4s(args, out_dtype, &a, &sp);
     if (st != hipSuccess) return st;
     const auto& x = *args;
-    const Mx4sRoute r = route_mx4s(x, kernel_id, workspace != nullptr);
+    const Mx4sRoute r = route_mx4s(x, kernel_id, workspace != nullptr, workspace_bytes);
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -1873,6 +2099,15 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
             }
             return qg::launch_slice_mx4s(ra, r.sl.mb, x.batch, bf16, stream);
         }
+        case QGEMM_KID_RING: {
+            qg::RingArgs ra = ring_args(r.rg, t, bf16, workspace);
+            ra.a_bytes = (long long)(x.m - 1) * x.stride_a + kb;
+            ra.b_bytes = (long long)x.n * kb;
+            ra.sfa_bytes = (long long)((x.m - 1) / 32) * x.stride_sfa + x.k;
+            ra.sfb_bytes = (long long)((x.n - 1) / 32) * x.stride_sfb + x.k;
+            st = qg::launch_ring_mx4s(ra, r.rg.mb, r.rg.nb, x.batch, stream);
+            return st != hipSuccess ? st : ring_reduce(ra, x.batch, bf16, stream);
+        }
         case QGEMM_KID_BURST: {
             qg::BurstArgs b{};
             b.t = t;
@@ -1897,7 +2132,7 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
 }
 size_t gemm_a4w4_mxfp4_bpreshuffle_kid_workspace_bytes(const opus_gemm_mxfp4_scale_kargs* args, int kernel_id) {
     if (!args || args->m <= 0 || args->n <= 0 || args->k <= 0 || args->k % 256 || args->batch <= 0) return 0;
-    const Mx4sRoute r = route_mx4s(*args, kernel_id, true);
+    const Mx4sRoute r = route_mx4s(*args, kernel_id, true, SIZE_MAX);
     return r.ok ? r.ws_bytes : 0;
 }
 hipError_t gemm_a4w4_mxfp4_bpreshuffle(const opus_gemm_mxfp4_scale_kargs* args, int out_dtype, hipStream_t stream) {
@@ -2079,7 +2314,8 @@ hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int
     if (a.batch > 1 && ((long long)a.stride_b_batch < bk || a.stride_b_batch % 16)) return hipErrorInvalidValue;
     sp.add(a.ptr_b, span(a.batch, a.stride_b_batch, 1, 0, bk, 1));
     if (sp.overlap_any(sp.p[0], sp.bytes[0], sp.n - 1)) return hipErrorInvalidValue;
-    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bk, false, kernel_id, workspace != nullptr);
+    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bk, false, kernel_id, workspace != nullptr,
+                                   workspace_bytes);
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -2097,7 +2333,7 @@ hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int
 size_t gemm_a8w8_blockscale_bpreshuffle_kid_workspace_bytes(const opus_gemm_kargs* args, int kernel_id) {
     if (!args || args->k <= 0 || args->k % 128) return 0;
     const BsfRoute r = route_bsf32(args->m, args->n, args->k / 128, args->batch, (long long)args->n * args->k, false,
-                                   kernel_id, true);
+                                   kernel_id, true, SIZE_MAX);
     return r.ok ? r.ws_bytes : 0;
 }
 
@@ -2128,7 +2364,8 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_kid(const opus_gemm_ldsbypass_kargs* a
     // decode shapes: the burst kernel (B'' fragments straight into
     // registers); other small M: the skinny kernel streams B'' into
     // registers; large M: the tile kernels stage B'' blocks through LDS
-    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bpp, true, kernel_id, workspace != nullptr);
+    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bpp, true, kernel_id, workspace != nullptr,
+                                   workspace_bytes);
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -2146,7 +2383,7 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_kid(const opus_gemm_ldsbypass_kargs* a
 size_t gemm_a8w8_blockscale_ldsbypass_kid_workspace_bytes(const opus_gemm_ldsbypass_kargs* args, int kernel_id) {
     if (!args || args->k <= 0 || args->k % 128 || args->n <= 0) return 0;
     const BsfRoute r = route_bsf32(args->m, args->n, args->k / 128, args->batch,
-                                   (long long)frag_bytes(args->n, args->k), true, kernel_id, true);
+                                   (long long)frag_bytes(args->n, args->k), true, kernel_id, true, SIZE_MAX);
     return r.ok ? r.ws_bytes : 0;
 }
 

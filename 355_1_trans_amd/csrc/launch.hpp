@@ -103,6 +103,13 @@ hipError_t launch_slice(const RunsArgs& a, bool fp4, int mb, int batch, bool bf1
 // the same for MXFP4 in aiter's formats: W16 B (b_bytes = N * K / 2) and
 // e8m0_shuffle scales (sfa_sm / sfb_sn = bytes per 32-row block)
 hipError_t launch_slice_mx4s(const RunsArgs& a, int mb, int batch, bool bf16, hipStream_t s);
+// kernels_ring_mx.hip / kernels_ring_bs.hip: ring decode kernel (M <= 16 mb, 16 nb
+// columns per workgroup; (mb, nb) in {1, 2} x {1, 2, 4} or 4 x {1, 2}); panel:
+// scales as 16 / 32 bytes per row and stage.  A split's slice sum is the caller's.
+struct RingArgs;
+hipError_t launch_ring_mx(const RingArgs& a, bool fp4, int mb, int nb, bool panel, int batch, hipStream_t s);
+hipError_t launch_ring_bs(const RingArgs& a, bool frag, int mb, int nb, bool panel, int batch, hipStream_t s);
+hipError_t launch_ring_mx4s(const RingArgs& a, int mb, int nb, int batch, hipStream_t s);
 // B' (K-panel) -> B'' (fragment order of the LDS-bypass path)
 hipError_t launch_repack_frag(const uint8_t* bk, uint8_t* bpp, int n, int k, int batch, long long bk_batch,
                               long long bpp_batch, hipStream_t s);

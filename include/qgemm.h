@@ -190,6 +190,10 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_repack(const opus_gemm_ldsbypass_kargs
                                 straight from memory, 32 / 64 / 128 columns per workgroup for M <= 16 /
                                 32 / 64; row-major entries: 16-byte aligned A / B rows and scale rows;
                                 also the aiter-format MXFP4 entry (W16 B, e8m0_shuffle scales) */
+#define QGEMM_KID_RING   11  /* ring decode kernel (M <= 64): DMA waves stream B and A through an LDS ring
+                                beside the MFMA waves; fp32 block scales, MX (16-byte aligned A / B rows,
+                                dword-aligned scale rows) and the aiter-format MXFP4 entry; a K split only
+                                with the workspace */
 hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int out_dtype, int kernel_id,
                                                 void* workspace, size_t workspace_bytes, hipStream_t stream);
 size_t gemm_a8w8_blockscale_bpreshuffle_kid_workspace_bytes(const opus_gemm_kargs* args, int kernel_id);
@@ -285,11 +289,12 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle(const opus_gemm_mxfp4_scale_kargs* args, 
  * kernel, or the two-by-two wave kernel for grid_blocks > 0),
  * QGEMM_KID_TILE256 (the two-by-two wave 256x256 tile kernel, the only one
  * that takes grid_blocks > 0), QGEMM_KID_QUAD (one-by-four waves, B straight
- * from memory into registers), QGEMM_KID_BURST (M <= 64) or QGEMM_KID_SLICE
- * (M <= 64: A's K slice in LDS, B's W16 fragments straight into registers);
- * other ids, and shapes a forced id cannot take, are rejected.  The
+ * from memory into registers), QGEMM_KID_BURST (M <= 64), QGEMM_KID_SLICE
+ * (M <= 64: A's K slice in LDS, B's W16 fragments straight into registers) or
+ * QGEMM_KID_RING (M <= 64: through an LDS ring filled by DMA waves); other ids, and shapes a forced id cannot take, are rejected.  The
  * workspace (size from the query below, 256-byte aligned, any contents)
- * carries a burst or slice plan's split-K counters and fp32 partials; the
+ * carries a burst or slice plan's split-K counters and fp32 partials (a ring
+ * plan's partials); the
  * plain entry above runs without one. */
 hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* args, int out_dtype, int kernel_id,
                                            void* workspace, size_t workspace_bytes, hipStream_t stream);
