@@ -460,35 +460,55 @@ __global__ __launch_bounds__(256) void quant_wgt_block_kernel(const QuantArgs p)
 }
 
 // ---------------------------------------------------------------- layouts
-// Every layout kernel walks its DESTINATION in order, one 16-byte unit per
-// thread (coalesced stores), and gathers the source unit.
+// K-panel [kt][n][128]; W16 [n/16][kbytes/16][16 rows][16] and FRAG, the same
+// order with the rows padded by zeros to a multiple of 16 (per K-tile
+// [h][q][row][16], chunk 4 h + q).
+//
+// A workgroup moves 16 rows x 2 U K-tiles, a thread U units of 16 bytes, all
+// loads before the stores.  A wave's 64 units are 8 rows x one K-tile: whole
+// 128-byte lines on both sides.  W16 / FRAG stores go through LDS, so that
+// neighbouring lanes store neighbouring rows of a chunk (stored as loaded:
+// 1.05-1.09x the time).  Every byte is touched once: nontemporal both ways
+// (1.06-1.2x).  HBM-bound: walking the destination unit by unit, reading half
+// lines -> this, us, N x K bytes: W16 and FRAG 7168 x 8192 23.8 -> 20.7, 4096 x
+// 7168 14.5 -> 11.9, 2112 x 7168 9.0 -> 7.0, 16384 x 6144 40.2 -> 33.8 (6.0
+// TB/s; a 1 GiB device copy 5.0); KPANEL 25.1 -> 22.7, 14.6 -> 13.0, 9.1 ->
+// 7.1, 39.7 -> 35.3; 1536 x 2048 3.4 -> 3.1.
 enum class Lay : int { KPANEL = 0, W16 = 1, FRAG = 2 };
 
-template <Lay L>
+template <Lay L, int U>
 __global__ __launch_bounds__(256) void relayout_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                                        int n, int kbytes, long long ld) {
-    const long long units = (L == Lay::FRAG ? (long long)((n + 15) / 16) * 16 : (long long)n) * (kbytes / 16);
-    for (long long u = (long long)blockIdx.x * 256 + threadIdx.x; u < units; u += (long long)gridDim.x * 256) {
-        long long so;
-        bool zero = false;
-        if constexpr (L == Lay::KPANEL) {            // dst [kt][n][8 chunks]
-            const long long kt = u / ((long long)n * 8), rem = u - kt * n * 8;
-            so = (rem >> 3) * ld + kt * 128 + (rem & 7) * 16;
-        } else if constexpr (L == Lay::W16) {        // dst [n/16][kbytes/16][16 rows][16]
-            const long long per_blk = (long long)(kbytes / 16) * 16;
-            const long long nb = u / per_blk, rem = u - nb * per_blk;
-            so = (nb * 16 + (rem & 15)) * ld + (rem >> 4) * 16;
-        } else {                                     // dst [n/16][kbytes/128][h][lane][16]
-            const int nkt = kbytes / 128;
-            const int lane = (int)(u & 63), h = (int)((u >> 6) & 1);
-            const long long blk = u >> 7, nb = blk / nkt, kt = blk - nb * nkt;
-            const long long row = nb * 16 + (lane & 15);
-            zero = row >= n;
-            so = row * ld + kt * 128 + ((lane >> 4) + 4 * h) * 16;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = (w & 1) * 8 + (lane >> 3), chunks = kbytes / 16;
+    const int c0 = (blockIdx.x * 2 * U + (w >> 1)) * 8 + (lane & 7);    // chunk of unit 0; unit i: + 16 i
+    __shared__ i32x4 turn[L == Lay::KPANEL ? 1 : 256];
+    i32x4* const mine = turn + w * 64;
+    const int blocks = n / 16 + (n % 16 != 0);
+    for (int nb = blockIdx.y; nb < blocks; nb += gridDim.y) {
+        const long long row = (long long)nb * 16 + r;
+        if (L != Lay::FRAG && row >= n) continue;
+        const uint8_t* const in = src + row * ld;
+        i32x4 v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            v[i] = i32x4{0, 0, 0, 0};
+            if (row < n && c0 + 16 * i < chunks) v[i] = __builtin_nontemporal_load((const i32x4*)(in + (c0 + 16 * i) * 16LL));
         }
-        i32x4 v = {0, 0, 0, 0};
-        if (!zero) v = *(const i32x4*)(src + so);
-        *(i32x4*)(dst + u * 16) = v;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            if constexpr (L == Lay::KPANEL) {
+                const int c = c0 + 16 * i;
+                if (c < chunks) __builtin_nontemporal_store(v[i], (i32x4*)(dst + ((long long)(c >> 3) * n + row) * 128 + (c & 7) * 16));
+            } else {    // through LDS, so that neighbouring lanes hold neighbouring rows of one chunk
+                mine[lane ^ (lane >> 3)] = v[i];
+                __builtin_amdgcn_wave_barrier();
+                const i32x4 x = mine[((lane & 7) * 8 + (lane >> 3)) ^ (lane & 7)];
+                __builtin_amdgcn_wave_barrier();
+                const int c = c0 - (lane & 7) + (lane >> 3) + 16 * i;
+                if (c < chunks) __builtin_nontemporal_store(x, (i32x4*)(dst + ((long long)nb * chunks + c) * 256 + ((w & 1) * 8 + (lane & 7)) * 16));
+            }
+        }
     }
 }
 
@@ -637,14 +657,21 @@ hipError_t launch_quant_wgt_blocks(int fmt, bool bf16in, const void* w, long lon
     return hipErrorInvalidValue;
 }
 
+template <Lay L>
+static void relayout_go(const uint8_t* src, uint8_t* dst, int n, int kbytes, long long ld, hipStream_t st) {
+    const int blocks = n / 16 + (n % 16 != 0), kt = kbytes / 128 + (kbytes % 128 != 0);
+    const unsigned y = blocks < 65535 ? blocks : 65535;
+    // four units per thread once 2048 workgroups of them remain, one where the
+    // chip would stand idle
+    if ((long long)blocks * kt >= 16384) relayout_kernel<L, 4><<<dim3((kt + 7) / 8, y), 256, 0, st>>>(src, dst, n, kbytes, ld);
+    else relayout_kernel<L, 1><<<dim3((kt + 1) / 2, y), 256, 0, st>>>(src, dst, n, kbytes, ld);
+}
 hipError_t launch_relayout(int layout, const uint8_t* src, uint8_t* dst, int n, int kbytes, long long ld,
                            hipStream_t st) {
-    const long long units = (layout == 2 ? (long long)((n + 15) / 16) * 16 : (long long)n) * (kbytes / 16);
-    const unsigned grid = grid_for(units);
     switch (layout) {
-        case 0: relayout_kernel<Lay::KPANEL><<<grid, 256, 0, st>>>(src, dst, n, kbytes, ld); trace_launch("relayout<KPANEL>"); break;
-        case 1: relayout_kernel<Lay::W16><<<grid, 256, 0, st>>>(src, dst, n, kbytes, ld); trace_launch("relayout<W16>"); break;
-        case 2: relayout_kernel<Lay::FRAG><<<grid, 256, 0, st>>>(src, dst, n, kbytes, ld); trace_launch("relayout<FRAG>"); break;
+        case 0: relayout_go<Lay::KPANEL>(src, dst, n, kbytes, ld, st); trace_launch("relayout<KPANEL>"); break;
+        case 1: relayout_go<Lay::W16>(src, dst, n, kbytes, ld, st); trace_launch("relayout<W16>"); break;
+        case 2: relayout_go<Lay::FRAG>(src, dst, n, kbytes, ld, st); trace_launch("relayout<FRAG>"); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
