@@ -2707,7 +2707,14 @@ double group_cost(const GroupProblem* p, int count, int nb, const int* splitk, c
 // splits of the problem whose items stream the most bytes while the cost
 // model drops by at least 1%.  Workspace: the split problems' counter words
 // (one per tile), then each split problem's fp32 partial planes.
-GroupPlan plan_grouped(const GroupProblem* p, int count, bool mx, bool frag, int cus, bool allow_split) {
+//
+// `lean`: fp32 scales at M = 17-32 take at most two K-tiles per wave in 16-wave
+// 32 x 32 tiles, as the MX formats do: four spill (the 128 VGPRs of a 16-wave
+// workgroup; the trio at M = 32 51.6 us, with two 25.4), and 16-column tiles
+// only where 32-column ones leave CUs idle or need a split without a workspace
+// (the trio unsplit on them 30.6 - 37.5 us at M = 17 - 32).  The plan without
+// it stays for calls whose workspace holds no other.
+GroupPlan plan_grouped(const GroupProblem* p, int count, bool mx, bool frag, int cus, bool allow_split, bool lean) {
     GroupPlan best;
     if (count < 1 || count > qg::kGroupMax) return best;
     int mmax = 0;
@@ -2720,9 +2727,14 @@ GroupPlan plan_grouped(const GroupProblem* p, int count, bool mx, bool frag, int
     // twice the waves' loads in flight per item wins -- configs[2]'s decode
     // trio, fp32 block scales, M = 1 / 16: 18.3 / 21.1 us with 8 waves x 8
     // K-tiles, 17.5 / 19.2 us with 16 x 4
-    for (int nb : {2, 1})
+    for (int nb : {2, 1}) {
+        if (lean && !mx && mb == 2 && nb == 1 && best.ok) {
+            int items = 0;
+            for (int j = 0; j < count; ++j) items += best.n_tiles[j] * best.splitk[j];
+            if (items >= cus) break;
+        }
         for (int waves : {16, 8}) {
-            const int kmax = qg::burst_max_kpw(mb, nb, waves, mx);
+            const int kmax = qg::burst_max_kpw(mb, nb, waves, mx || lean);
             if (kmax == 0 || qg::burst_lds_bytes(mb, nb, waves, !frag) > qg::kBurstLdsMax) continue;
             const int cap = waves * kmax;
             GroupPlan c;
@@ -2771,6 +2783,7 @@ GroupPlan plan_grouped(const GroupProblem* p, int count, bool mx, bool frag, int
                 best = c;
             }
         }
+    }
     if (!best.ok) return best;
     size_t ctr = 0, part = 0;
     best.items = 0;
@@ -2876,9 +2889,21 @@ hipError_t group_collect(GroupFam fam, const void* kargs, int count, int out_dty
     return hipSuccess;
 }
 
-GroupPlan group_plan(GroupFam fam, const GroupCall& g, bool allow_split) {
-    return plan_grouped(g.shape, g.count, fam == GroupFam::MX8 || fam == GroupFam::MX4, fam == GroupFam::BS_FRAG,
-                        device_cus(), allow_split);
+GroupPlan group_plan(GroupFam fam, const GroupCall& g, bool have_ws, size_t ws_cap) {
+    const bool mx = fam == GroupFam::MX8 || fam == GroupFam::MX4, frag = fam == GroupFam::BS_FRAG;
+    auto plan = [&](bool split, bool lean) {
+        return plan_grouped(g.shape, g.count, mx, frag, device_cus(), split, lean);
+    };
+    if (have_ws) {
+        const GroupPlan p = plan(true, true);
+        if (p.ok && p.ws_bytes <= ws_cap) return p;
+    }
+    const GroupPlan old = plan(have_ws, false);
+    if (old.ok && old.ws_bytes == 0) {    // fits as it is: unsplit, and lean if that can be
+        const GroupPlan p = plan(false, true);
+        if (p.ok) return p;
+    }
+    return old;
 }
 
 hipError_t group_entry(GroupFam fam, const void* kargs, int count, int out_dtype, int grid_blocks, void* ws,
@@ -2889,7 +2914,7 @@ hipError_t group_entry(GroupFam fam, const void* kargs, int count, int out_dtype
     int span_begin[qg::kGroupMax + 1];
     hipError_t st = group_collect(fam, kargs, count, out_dtype, &g, span_begin);
     if (st != hipSuccess) return st;
-    const GroupPlan pl = group_plan(fam, g, ws != nullptr);
+    const GroupPlan pl = group_plan(fam, g, ws != nullptr, aligned(ws, 256) ? ws_bytes : 0);
     if (!pl.ok) return hipErrorInvalidValue;
     if (ws && pl.ws_bytes) {
         if (ws_bytes < pl.ws_bytes || !aligned(ws, 256)) return hipErrorInvalidValue;
@@ -2938,7 +2963,7 @@ size_t group_workspace(GroupFam fam, const void* kargs, int count) {
     GroupCall g;
     int span_begin[qg::kGroupMax + 1];
     if (group_collect(fam, kargs, count, QGEMM_OUT_BF16, &g, span_begin) != hipSuccess) return 0;
-    const GroupPlan pl = group_plan(fam, g, true);
+    const GroupPlan pl = group_plan(fam, g, true, SIZE_MAX);
     return pl.ok ? pl.ws_bytes : 0;
 }
 

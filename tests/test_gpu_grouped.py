@@ -122,3 +122,21 @@ def test_grouped_sixteen_problems(qgemm, gpu):
     assert ",g16," in trace, trace
     for (m, n, k), ref, y in zip(shapes, refs, ys):
         assert_close(ref, out_to_f32(y), f"mxfp4 grouped {m}x{n}x{k} ({trace})")
+
+
+@pytest.mark.parametrize("kind", ["bpreshuffle", "ldsbypass"])
+@pytest.mark.parametrize("m", [17, 32])
+def test_grouped_two_row_blocks_long_k(qgemm, gpu, kind, m):
+    """fp32 scales at M = 17-32: no 16-wave 32 x 32 tiles of four K-tiles per
+    wave (they spill), with a workspace for a K split, without one, or with
+    one too small for it."""
+    shapes = [(m, n, k) for n, k in C2_DECODE]
+    probs, refs = _problems(qgemm, gpu, kind, shapes, seed=23)
+    small = torch.full((512,), 0xFF, dtype=torch.uint8, device=gpu)
+    for ws in (None, False, small):
+        ys = qgemm.gemm_grouped(kind, probs, workspace=ws)
+        trace = qgemm.last_launch()
+        torch.cuda.synchronize()
+        assert ",nb2,w16,kpw4," not in trace, trace
+        for (mm, n, k), ref, y in zip(shapes, refs, ys):
+            assert_close(ref, out_to_f32(y), f"{kind} grouped {mm}x{n}x{k} ({trace})")
