@@ -733,6 +733,14 @@ BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bo
     return r;
 }
 
+// MX, M > 1024 and at most kMidBelow 256 x 256 tiles: the 128 x 128 kernel to 64
+// K-tiles (M = 2048 - 4096, N = 1536 - 4096: MXFP8 K = 4096 41-46 -> 33-37 us,
+// K = 7168 56-68 -> 46-58 against the 256 x 256 kernel with its K split, MXFP4
+// 27-31 -> 23-25 and 39-44 -> 33-37; at 80 K-tiles MXFP8 equal, at 128 1.04-1.1x
+// slower).  From 136 tiles on the 256 x 256 kernel is 1.1-1.35x faster.  M <=
+// 1024 measured alike; its routes are pinned by tests and stay.
+bool mid_mx_deep(int m, int k_tiles) { return m > 1024 && k_tiles <= 64; }
+
 // MX: the same 128 x 128 rule (row-major B, E8M0 scales applied by the
 // MFMA); small M on >= 128 256 x 256 tiles runs the 128 x 128 kernel
 // (N = 32768 - 129280, MXFP4 / MXFP8 M = 24-128: 1.1-1.7x over the
@@ -750,9 +758,9 @@ Plan plan_mx(int m, int n, int k_tiles, int batch, long long b_bytes, bool fp4) 
     // fp4); longer K from 96 tiles runs the 256 x 256 kernel (M = 512-1024,
     // N = 6144-12288, K = 2048-7168: 128 x 128 1.03-1.2x slower there,
     // 1.1-1.3x faster with short K; N = 8192, M = 1024, K = 1536 MXFP4
-    // 18.6 -> 14.0 us)
+    // 18.6 -> 14.0 us); M > 1024 up to 64 K-tiles (mid_mx_deep)
     const long long tiles256 = (long long)ceil_div(m, 256) * ceil_div(n, 256) * batch;
-    const bool short_k = k_tiles <= (fp4 ? 12 : 16);
+    const bool short_k = k_tiles <= (fp4 ? 12 : 16) || mid_mx_deep(m, k_tiles);
     if (m <= 256 || tiles256 < 96 || (tiles256 <= kMidBelow && short_k))
         plan_mid(p, m, n, k_tiles, batch, cus, m > 256 && tiles256 == kMidBelow);
     if (!p.skinny && !p.mid && small_m_wide(m, n, batch, (long long)k_tiles * (fp4 ? 256 : 128), cus)) {
@@ -1401,7 +1409,7 @@ MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws
             r.pl = plan_mx(a.m, a.n, kt, a.batch, bb, fp4);
             r.sp = plan_stream(a.m, a.n, a.k, a.batch, fp4);
             r.bp = plan_mx_burst(a.m, a.n, kt, a.batch, true);
-            if (r.pl.mid && a.m > 128 && have_ws) {
+            if (r.pl.mid && a.m > 128 && !mid_mx_deep(a.m, kt) && have_ws) {
                 // M > 128 on a 128 x 128 plan: the four-wave kernel's K
                 // split where its slices fill >= 9/16 of the CUs (M = 512 /
                 // 768, N = 6144 / 8192, K = 12288 / 16384: 1.4-1.6x over the

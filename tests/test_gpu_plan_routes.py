@@ -135,3 +135,15 @@ def test_mx8_wide_split_variants(qgemm, gpu, case):
     rows, cols = _points(m, n, m + n + k)
     ref = O.gemm_mx8_points(_host(A), _host(B), _host(SA), _host(SB), rows, cols)
     assert_close(ref, y.float().cpu().numpy()[rows, cols], f"mx8 {m}x{n}x{k} {case} ({trace})")
+
+
+@pytest.mark.parametrize("fam,m,n,k,expect", [
+    ("mx8", 1025, 5130, 8192, "mid_gemm<fp8,MX"),                    # 105 tiles, 64 K-tiles
+    ("mx8", 1025, 5130, 8320, "wide_gemm<fp8,MX"),                   # 65 K-tiles
+    ("mx4", 1040, 6400, 3328, "mid_gemm<fp4,MX"),                    # 125 tiles, 13 K-tiles
+    ("mx8", 2048, 4096, 2176, "mid_gemm<fp8,MX"),                    # 128 tiles
+    ("mx4", 1040, 6660, 4096, "mx_scale_panels<pb32>+wide_gemm"),    # 135 tiles
+])
+def test_mx_long_k_past_1024_rows(qgemm, gpu, fam, m, n, k, expect):
+    """M > 1024 on at most 128 tiles of 256 x 256: the 128 x 128 kernel to 64 K-tiles."""
+    test_mx_plan_route(qgemm, gpu, fam, m, n, k, expect)
