@@ -472,8 +472,8 @@ __global__ __launch_bounds__(256) void quant_wgt_block_kernel(const QuantArgs p)
 // (1.06-1.2x).  HBM-bound: walking the destination unit by unit, reading half
 // lines -> this, us, N x K bytes: W16 and FRAG 7168 x 8192 23.8 -> 20.7, 4096 x
 // 7168 14.5 -> 11.9, 2112 x 7168 9.0 -> 7.0, 16384 x 6144 40.2 -> 33.8 (6.0
-// TB/s; a 1 GiB device copy 5.0); KPANEL 25.1 -> 22.7, 14.6 -> 13.0, 9.1 ->
-// 7.1, 39.7 -> 35.3; 1536 x 2048 3.4 -> 3.1.
+// TB/s; a 1 GiB device copy 5.0); KPANEL 25.1 -> 22.7, 14.6 -> 10.9, 9.1 ->
+// 6.5, 39.7 -> 35.3; 1536 x 2048 3.4 -> 3.1.
 enum class Lay : int { KPANEL = 0, W16 = 1, FRAG = 2 };
 
 template <Lay L, int U>
@@ -661,9 +661,10 @@ template <Lay L>
 static void relayout_go(const uint8_t* src, uint8_t* dst, int n, int kbytes, long long ld, hipStream_t st) {
     const int blocks = n / 16 + (n % 16 != 0), kt = kbytes / 128 + (kbytes % 128 != 0);
     const unsigned y = blocks < 65535 ? blocks : 65535;
-    // four units per thread once 2048 workgroups of them remain, one where the
-    // chip would stand idle
-    if ((long long)blocks * kt >= 16384) relayout_kernel<L, 4><<<dim3((kt + 7) / 8, y), 256, 0, st>>>(src, dst, n, kbytes, ld);
+    // four units per thread once 2048 workgroups of them remain, K-panel 512
+    // (4096 x 7168 12.9 -> 10.9 us, 7168 x 2048 7.2 -> 6.3, 2112 x 7168 6.9 -> 6.5;
+    // W16 / FRAG there 0.96-1.05x); else one
+    if ((long long)blocks * kt >= (L == Lay::KPANEL ? 4096 : 16384)) relayout_kernel<L, 4><<<dim3((kt + 7) / 8, y), 256, 0, st>>>(src, dst, n, kbytes, ld);
     else relayout_kernel<L, 1><<<dim3((kt + 1) / 2, y), 256, 0, st>>>(src, dst, n, kbytes, ld);
 }
 hipError_t launch_relayout(int layout, const uint8_t* src, uint8_t* dst, int n, int kbytes, long long ld,

@@ -13,8 +13,8 @@ def _source(n, k, pad, gpu):
     return torch.randint(0, 256, (n, k + pad), dtype=torch.uint8, generator=g, device=gpu)[:, :k]
 
 
-# 16384 row blocks x K-tiles is where the larger workgroups begin
-SIZES = [(16, 128), (48, 384), (80, 1152), (4096, 8064), (4096, 8192), (4112, 9344)]
+# 16384 row blocks x K-tiles is where the larger workgroups begin, 4096 for K-panel
+SIZES = [(16, 128), (48, 384), (80, 1152), (1024, 8064), (1024, 8192), (4096, 8064), (4096, 8192), (4112, 9344)]
 
 
 @pytest.mark.parametrize("pad", [0, 16])
