@@ -210,7 +210,7 @@ static_assert(kSplitBelow <= kMaxCounters, "counter block too small");
 // a counter word held before: a workspace needs no clearing, and one left
 // mid-count (an interrupted launch) or never zeroed cannot make a slice
 // take itself for the last.  Launches that share a workspace are
-// stream-ordered, so consecutive epochs never meet on one word.
+// stream-ordered (workspace_turn), so consecutive epochs never meet on one word.
 std::atomic<unsigned> g_epoch{0};
 unsigned next_epoch() { return (g_epoch.fetch_add(1u, std::memory_order_relaxed) + 1u) & 0xffffffu; }
 // the counter word's arrival count is 8 bits: no plan splits K more ways
@@ -1694,6 +1694,18 @@ hipError_t check_workspace(const void* ws, size_t ws_bytes, size_t need, const S
     return hipSuccess;
 }
 
+// A call's turn at its workspace, held over its launches (nothing without
+// one): the launches of a plan with several -- partial planes or a scale copy,
+// then the kernel that reads them -- follow each other on the stream with no
+// launch of another thread's call on the same workspace between them.  The
+// mutexes are shared by address; a call holds one.
+std::mutex g_turn_mu[64];
+std::unique_lock<std::mutex> workspace_turn(const void* ws) {
+    if (!ws) return {};
+    const uint64_t h = (reinterpret_cast<uintptr_t>(ws) >> 8) * 0x9E3779B97F4A7C15ull;
+    return std::unique_lock<std::mutex>(g_turn_mu[h >> 58]);
+}
+
 // Validation shared by the MX entry points: dense or padded row-major A/B,
 // row-major scales, C [M, N] with stride_c >= N.
 hipError_t validate_mx(const opus_gemm_scale_kargs* args, int out_dtype, int kbytes_per_row, int k_align,
@@ -1821,6 +1833,7 @@ static hipError_t mx_entry(const opus_gemm_scale_kargs* args, bool fp4, int out_
     fill_common(t, a, fp4 ? a.k / 2 : a.k, out_dtype ? 2 : 4);
     t.sfa_sm = a.stride_sfa;
     t.sfb_sn = a.stride_sfb;
+    const auto turn = workspace_turn(workspace);
     return run_mx(r, t, a, fp4, out_dtype == QGEMM_OUT_BF16, workspace, workspace_bytes, stream);
 }
 
@@ -2063,6 +2076,7 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
     t.sfa_sm = x.stride_sfa;
     t.sfb_sn = x.stride_sfb;
     t.sfa_sk = t.sfb_sk = 256;
+    const auto turn = workspace_turn(workspace);
     switch (r.kid) {
         case QGEMM_KID_QUAD: {
             if (r.qsplit <= 1) return qg::launch_quad_mx4(t, x.batch, true, bf16, stream);
@@ -2334,6 +2348,7 @@ hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int
     t.sfa_sm = sfa_sm;
     t.sfa_sk = sfa_sk;
     t.sfb_sn = a.stride_sfb;
+    const auto turn = workspace_turn(workspace);
     return run_bsf32(r, t, a.batch, false, bk, out_dtype == QGEMM_OUT_BF16, workspace, workspace_bytes, a.k / 128,
                      stream);
 }
@@ -2384,6 +2399,7 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_kid(const opus_gemm_ldsbypass_kargs* a
     t.sfa_sm = sfa_sm;
     t.sfa_sk = sfa_sk;
     t.sfb_sn = a.stride_sfb;
+    const auto turn = workspace_turn(workspace);
     return run_bsf32(r, t, a.batch, true, bpp, out_dtype == QGEMM_OUT_BF16, workspace, workspace_bytes, a.k / 128,
                      stream);
 }
@@ -2931,6 +2947,7 @@ hipError_t group_entry(GroupFam fam, const void* kargs, int count, int out_dtype
     }
     st = check_arch();
     if (st != hipSuccess) return st;
+    const auto turn = workspace_turn(ws);
     qg::BurstGroup bg{};
     bg.count = count;
     const unsigned epoch = next_epoch();

@@ -147,7 +147,9 @@ size_t gemm_a8w8_blockscale_layout_workspace_bytes(const opus_gemm_scale_kargs* 
  * the queried bytes, 256-byte aligned, any contents; its first 2048 bytes
  * are arrival counters that each launch tags with a fresh epoch, so they
  * need no clearing (a completed call leaves them zero).  Calls that share a
- * workspace must be ordered (same stream).  The MX entries' plan, and so
+ * workspace must be on one stream; they may come from several threads (a
+ * call's launches -- some plans sum partial planes in a second one -- are
+ * queued together, whatever other threads queue).  The MX entries' plan, and so
  * the rounding of their last bits, also depends on workspace_bytes: the
  * four-wave kernel's K split is taken only when its planes fit (a workspace
  * of at least the scale-panel bytes but less than the query runs unsplit). */
