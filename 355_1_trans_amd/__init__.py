@@ -247,6 +247,18 @@ def _require_gpu(*tensors):
 _WORKSPACES = {}
 
 
+class _Address(int):
+    """The address of a cached buffer, which it keeps alive: another thread's
+    call may put a larger buffer in its place before the launch is queued
+    (after it, memory that goes back to the allocator is reused in stream
+    order)."""
+
+    def __new__(cls, buf):
+        self = super().__new__(cls, buf.data_ptr())
+        self.buf = buf
+        return self
+
+
 def _workspace(query, args, workspace, dev, stream):
     """(pointer, bytes) of the split-K workspace for this call.
 
@@ -267,7 +279,7 @@ def _workspace(query, args, workspace, dev, stream):
     if buf is None or buf.numel() < need:
         buf = torch.zeros((need + 255) // 256 * 256, dtype=torch.uint8, device=dev)
         _WORKSPACES[key] = buf
-    return buf.data_ptr(), buf.numel()
+    return _Address(buf), buf.numel()
 
 
 def _ws_tensor(workspace):

@@ -26,7 +26,7 @@ from pathlib import Path
 
 import torch
 
-from . import Kargs, _check, _out_code, _record, _require_gpu, _stream, lib, shuffle_b_kpanel
+from . import Kargs, _Address, _check, _out_code, _record, _require_gpu, _stream, lib, shuffle_b_kpanel
 
 CONFIGS = Path(__file__).resolve().parent / "configs"
 
@@ -49,7 +49,7 @@ def _scratch(tag, need, dev, stream):
     if buf is None or buf.numel() < need:
         buf = torch.zeros((need + 255) // 256 * 256, dtype=torch.uint8, device=dev)
         _WS[key] = buf
-    return buf.data_ptr(), buf.numel()
+    return _Address(buf), buf.numel()
 
 
 def _cu_num(dev):

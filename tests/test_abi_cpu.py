@@ -348,6 +348,27 @@ def test_noalloc_plans_as_the_query(qgemm):
         assert L.gemm_a4w4_mxfp4_noalloc(ctypes.byref(fit), 1, None) != HIP_INVALID_VALUE
 
 
+def test_cached_workspace_outlives_its_replacement(qgemm, monkeypatch):
+    """The address that a call takes from a workspace cache keeps its buffer
+    alive: another thread's larger call may replace it before the launch."""
+    import types
+    import weakref
+
+    opus, stream, dev = qgemm.opus, types.SimpleNamespace(cuda_stream=0), torch.device("cpu")
+    monkeypatch.setattr(qgemm, "_WORKSPACES", {})
+    monkeypatch.setattr(opus, "_WS", {})
+    for cache, take in ((qgemm._WORKSPACES, lambda need: qgemm._workspace(lambda a: need, qgemm.Kargs(), None, dev, stream)),
+                        (opus._WS, lambda need: opus._scratch("splitk", need, dev, stream))):
+        address, nbytes = take(1000)
+        first = weakref.ref(next(iter(cache.values())))
+        assert nbytes == 1024 and address == first().data_ptr()
+        assert ctypes.c_void_p.from_param(address) is not None
+        take(5000)
+        assert next(iter(cache.values())) is not first() and first() is not None
+        del address
+        assert first() is None
+
+
 # ----------------------------------------------------------------- grouped entries
 def _group(qgemm, shapes, fp4=False, bs=False):
     """An array of far-apart fake kargs blocks (never dereferenced)."""
