@@ -538,6 +538,47 @@ TailPlan plan_tail(int m, int n, int k_tiles, int batch, int cus) {
     return tp;
 }
 
+// Byte ranges of a call's operands (C first), for the overlap checks of the
+// output and of the workspace.
+struct Spans {
+    const void* p[6];
+    uint64_t bytes[6];
+    int n = 0;
+    void add(const void* q, uint64_t b) {
+        p[n] = q;
+        bytes[n++] = b;
+    }
+    bool overlap_any(const void* q, uint64_t b, int from) const {
+        for (int i = from; i < n; ++i)
+            if (overlaps(q, b, p[i], bytes[i])) return true;
+        return false;
+    }
+};
+
+// One workspace rule for every entry point and every route: NULL runs
+// without a workspace (no K split; wide MX kernels read row-major scales
+// directly); a non-NULL workspace must hold the bytes the entry's
+// *_workspace_bytes query returns, be 256-byte aligned and overlap neither C
+// nor an input.  Checked once, before routing.
+hipError_t check_workspace(const void* ws, size_t ws_bytes, size_t need, const Spans& sp) {
+    if (!ws || need == 0) return hipSuccess;
+    if (ws_bytes < need || !aligned(ws, 256) || sp.overlap_any(ws, need, 0)) return hipErrorInvalidValue;
+    return hipSuccess;
+}
+
+// A call's workspace as the routes see it (a query: none yet, any size).
+struct WorkspaceView {
+    bool have;
+    size_t cap;
+    const void* p = nullptr;
+    const Spans* sp = nullptr;
+    // a plan of `need` bytes could run on it
+    bool holds(size_t need) const {
+        return have && need <= cap && (!sp || check_workspace(p, cap, need, *sp) == hipSuccess);
+    }
+};
+constexpr WorkspaceView kAnyWorkspace{true, SIZE_MAX};
+
 // Ring kernel (ring_gemm.hpp): M <= 64, 16 mb rows and 16 nb columns per
 // workgroup, K slices of whole stages (4 K-tiles).  (nb, split) is the pair
 // with the least modelled time: a fixed part, the extra launch and the
@@ -583,11 +624,10 @@ RingPlan plan_ring(int m, int n, int kt, int batch, bool rows, bool fp4, int cus
     r.ws_bytes = r.splitk > 1 ? kCounterBytes + (size_t)r.splitk * batch * m * n * 4 : 0;
     return r;
 }
-// an AUTO call takes its ring plan when its split's planes fit the workspace
-// at hand (none: only unsplit plans); what fitted without it still runs
-bool ring_fits(const RingPlan& p, bool have_ws, size_t ws_cap) {
-    return p.ok && (p.splitk == 1 || (have_ws && p.ws_bytes <= ws_cap));
-}
+// an AUTO call takes its ring plan when its split's planes can go into the
+// workspace at hand (none: only unsplit plans); a call whose workspace is too
+// small, not aligned or on an operand runs, or is refused, as without this plan
+bool ring_fits(const RingPlan& p, const WorkspaceView& w) { return p.ok && (p.splitk == 1 || w.holds(p.ws_bytes)); }
 // the ring kernel's arguments but for the load ranges
 qg::RingArgs ring_args(const RingPlan& p, const TileArgs& t, bool bf16, void* ws) {
     qg::RingArgs a{};
@@ -662,8 +702,9 @@ bool ring_bsf32(int m, int n, int kt, int batch, bool frag) {
     return n <= 8192 && kt > 16 && kt <= (n <= 7168 ? 56 : 48);
 }
 
-BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bool frag, int kid, bool have_ws,
-                     size_t ws_cap) {
+BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bool frag, int kid,
+                     const WorkspaceView& w) {
+    const bool have_ws = w.have;
     BsfRoute r;
     r.kid = kid;
     if (m <= 0 || n <= 0 || k_tiles <= 0 || batch <= 0) return r;
@@ -672,7 +713,7 @@ BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bo
         case QGEMM_KID_AUTO: {
             if (ring_bsf32(m, n, k_tiles, batch, frag)) {
                 r.rg = plan_ring(m, n, k_tiles, batch, false, false, cus, true);
-                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                if (ring_fits(r.rg, w)) {
                     r.kid = QGEMM_KID_RING;
                     r.ws_bytes = r.rg.ws_bytes;
                     r.ok = true;
@@ -1388,7 +1429,9 @@ bool ring_mx(int m, int n, int kt, bool fp4) {
     return n <= 8192 && row >= 1536 && !(m > 40 && kt >= 64 && kt < 72 && (n <= 4096 || (fp4 && n > 6144)));
 }
 
-MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws, size_t ws_cap) {
+MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, const WorkspaceView& w) {
+    const bool have_ws = w.have;
+    const size_t ws_cap = w.cap;
     MxRoute r;
     r.kid = kid;
     if (a.m <= 0 || a.n <= 0 || a.k <= 0 || a.batch <= 0 || a.k % (fp4 ? 256 : 128)) return r;
@@ -1399,7 +1442,7 @@ MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, bool have_ws
         case QGEMM_KID_AUTO: {
             if (a.batch == 1 && ring_mx(a.m, a.n, kt, fp4) && ring_panels(a, fp4)) {
                 r.rg = plan_ring(a.m, a.n, kt, 1, true, fp4, cus, true);
-                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                if (ring_fits(r.rg, w)) {
                     r.kid = QGEMM_KID_RING;
                     r.ws_bytes = r.rg.ws_bytes;
                     r.ok = true;
@@ -1666,34 +1709,6 @@ hipError_t run_mx(const MxRoute& r, TileArgs t, const opus_gemm_scale_kargs& a, 
     }
 }
 
-// Byte ranges of a call's operands (C first), for the overlap checks of the
-// output and of the workspace.
-struct Spans {
-    const void* p[6];
-    uint64_t bytes[6];
-    int n = 0;
-    void add(const void* q, uint64_t b) {
-        p[n] = q;
-        bytes[n++] = b;
-    }
-    bool overlap_any(const void* q, uint64_t b, int from) const {
-        for (int i = from; i < n; ++i)
-            if (overlaps(q, b, p[i], bytes[i])) return true;
-        return false;
-    }
-};
-
-// One workspace rule for every entry point and every route: NULL runs
-// without a workspace (no K split; wide MX kernels read row-major scales
-// directly); a non-NULL workspace must hold the bytes the entry's
-// *_workspace_bytes query returns, be 256-byte aligned and overlap neither C
-// nor an input.  Checked once, before routing.
-hipError_t check_workspace(const void* ws, size_t ws_bytes, size_t need, const Spans& sp) {
-    if (!ws || need == 0) return hipSuccess;
-    if (ws_bytes < need || !aligned(ws, 256) || sp.overlap_any(ws, need, 0)) return hipErrorInvalidValue;
-    return hipSuccess;
-}
-
 // A call's turn at its workspace, held over its launches (nothing without
 // one): the launches of a plan with several -- partial planes or a scale copy,
 // then the kernel that reads them -- follow each other on the stream with no
@@ -1823,7 +1838,7 @@ static hipError_t mx_entry(const opus_gemm_scale_kargs* args, bool fp4, int out_
     hipError_t st = validate_mx(args, out_dtype, args ? (fp4 ? args->k / 2 : args->k) : 0, fp4 ? 256 : 128, &sp);
     if (st != hipSuccess) return st;
     const auto& a = *args;
-    const MxRoute r = route_mx(a, fp4, kernel_id, workspace != nullptr, workspace_bytes);
+    const MxRoute r = route_mx(a, fp4, kernel_id, {workspace != nullptr, workspace_bytes, workspace, &sp});
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -1837,11 +1852,9 @@ static hipError_t mx_entry(const opus_gemm_scale_kargs* args, bool fp4, int out_
     return run_mx(r, t, a, fp4, out_dtype == QGEMM_OUT_BF16, workspace, workspace_bytes, stream);
 }
 
-// ws_cap: the most workspace the caller can bring (the four-wave kernel's
-// K split is planned only when its partial planes fit)
-static size_t mx_workspace(const opus_gemm_scale_kargs* args, bool fp4, int kernel_id, size_t ws_cap = SIZE_MAX) {
+static size_t mx_workspace(const opus_gemm_scale_kargs* args, bool fp4, int kernel_id) {
     if (!args) return 0;
-    const MxRoute r = route_mx(*args, fp4, kernel_id, true, ws_cap);
+    const MxRoute r = route_mx(*args, fp4, kernel_id, kAnyWorkspace);
     return r.ok ? r.ws_bytes : 0;
 }
 
@@ -1930,7 +1943,8 @@ bool ring_mx4s(int m, int n, int kt) {
     return m > 32 && m <= 64 && n > 1536 && n <= 7168 && kt >= 24;
 }
 
-Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws, size_t ws_cap) {
+Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, const WorkspaceView& w) {
+    const bool have_ws = w.have;
     Mx4sRoute r;
     const int kt = x.k / 256;
     const int cus = device_cus();
@@ -1945,7 +1959,7 @@ Mx4sRoute route_mx4s(const opus_gemm_mxfp4_scale_kargs& x, int kid, bool have_ws
             r.ok = true;
             if (x.grid_blocks == 0 && x.batch == 1 && ring_mx4s(x.m, x.n, kt)) {
                 r.rg = plan_ring(x.m, x.n, kt, 1, false, true, cus, true);
-                if (ring_fits(r.rg, have_ws, ws_cap)) {
+                if (ring_fits(r.rg, w)) {
                     r.kid = QGEMM_KID_RING;
                     r.ws_bytes = r.rg.ws_bytes;
                     return r;
@@ -2063,7 +2077,7 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
     hipError_t st = validate_mx4s(args, out_dtype, &a, &sp);
     if (st != hipSuccess) return st;
     const auto& x = *args;
-    const Mx4sRoute r = route_mx4s(x, kernel_id, workspace != nullptr, workspace_bytes);
+    const Mx4sRoute r = route_mx4s(x, kernel_id, {workspace != nullptr, workspace_bytes, workspace, &sp});
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -2154,7 +2168,7 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* ar
 }
 size_t gemm_a4w4_mxfp4_bpreshuffle_kid_workspace_bytes(const opus_gemm_mxfp4_scale_kargs* args, int kernel_id) {
     if (!args || args->m <= 0 || args->n <= 0 || args->k <= 0 || args->k % 256 || args->batch <= 0) return 0;
-    const Mx4sRoute r = route_mx4s(*args, kernel_id, true, SIZE_MAX);
+    const Mx4sRoute r = route_mx4s(*args, kernel_id, kAnyWorkspace);
     return r.ok ? r.ws_bytes : 0;
 }
 hipError_t gemm_a4w4_mxfp4_bpreshuffle(const opus_gemm_mxfp4_scale_kargs* args, int out_dtype, hipStream_t stream) {
@@ -2336,8 +2350,8 @@ hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int
     if (a.batch > 1 && ((long long)a.stride_b_batch < bk || a.stride_b_batch % 16)) return hipErrorInvalidValue;
     sp.add(a.ptr_b, span(a.batch, a.stride_b_batch, 1, 0, bk, 1));
     if (sp.overlap_any(sp.p[0], sp.bytes[0], sp.n - 1)) return hipErrorInvalidValue;
-    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bk, false, kernel_id, workspace != nullptr,
-                                   workspace_bytes);
+    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bk, false, kernel_id,
+                                   {workspace != nullptr, workspace_bytes, workspace, &sp});
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -2356,7 +2370,7 @@ hipError_t gemm_a8w8_blockscale_bpreshuffle_kid(const opus_gemm_kargs* args, int
 size_t gemm_a8w8_blockscale_bpreshuffle_kid_workspace_bytes(const opus_gemm_kargs* args, int kernel_id) {
     if (!args || args->k <= 0 || args->k % 128) return 0;
     const BsfRoute r = route_bsf32(args->m, args->n, args->k / 128, args->batch, (long long)args->n * args->k, false,
-                                   kernel_id, true, SIZE_MAX);
+                                   kernel_id, kAnyWorkspace);
     return r.ok ? r.ws_bytes : 0;
 }
 
@@ -2387,8 +2401,8 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_kid(const opus_gemm_ldsbypass_kargs* a
     // decode shapes: the burst kernel (B'' fragments straight into
     // registers); other small M: the skinny kernel streams B'' into
     // registers; large M: the tile kernels stage B'' blocks through LDS
-    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bpp, true, kernel_id, workspace != nullptr,
-                                   workspace_bytes);
+    const BsfRoute r = route_bsf32(a.m, a.n, a.k / 128, a.batch, bpp, true, kernel_id,
+                                   {workspace != nullptr, workspace_bytes, workspace, &sp});
     if (!r.ok) return hipErrorInvalidValue;
     st = check_workspace(workspace, workspace_bytes, r.ws_bytes, sp);
     if (st != hipSuccess) return st;
@@ -2407,7 +2421,8 @@ hipError_t gemm_a8w8_blockscale_ldsbypass_kid(const opus_gemm_ldsbypass_kargs* a
 size_t gemm_a8w8_blockscale_ldsbypass_kid_workspace_bytes(const opus_gemm_ldsbypass_kargs* args, int kernel_id) {
     if (!args || args->k <= 0 || args->k % 128 || args->n <= 0) return 0;
     const BsfRoute r = route_bsf32(args->m, args->n, args->k / 128, args->batch,
-                                   (long long)frag_bytes(args->n, args->k), true, kernel_id, true, SIZE_MAX);
+                                   (long long)frag_bytes(args->n, args->k), true, kernel_id,
+                                   kAnyWorkspace);
     return r.ok ? r.ws_bytes : 0;
 }
 
@@ -2913,14 +2928,23 @@ hipError_t group_collect(GroupFam fam, const void* kargs, int count, int out_dty
     return hipSuccess;
 }
 
-GroupPlan group_plan(GroupFam fam, const GroupCall& g, bool have_ws, size_t ws_cap) {
+// the grouped entries' workspace rule (check_workspace's, over every problem's operands)
+bool group_holds(const GroupCall& g, const void* ws, size_t ws_bytes, size_t need) {
+    if (ws_bytes < need || !aligned(ws, 256)) return false;
+    for (int i = 0; i < g.spans; ++i)
+        if (overlaps(ws, need, g.span_p[i], g.span_b[i])) return false;
+    return true;
+}
+
+// ws NULL with have_ws: a query, any workspace
+GroupPlan group_plan(GroupFam fam, const GroupCall& g, bool have_ws, const void* ws, size_t ws_bytes) {
     const bool mx = fam == GroupFam::MX8 || fam == GroupFam::MX4, frag = fam == GroupFam::BS_FRAG;
     auto plan = [&](bool split, bool lean) {
         return plan_grouped(g.shape, g.count, mx, frag, device_cus(), split, lean);
     };
     if (have_ws) {
         const GroupPlan p = plan(true, true);
-        if (p.ok && p.ws_bytes <= ws_cap) return p;
+        if (p.ok && (!ws || p.ws_bytes == 0 || group_holds(g, ws, ws_bytes, p.ws_bytes))) return p;
     }
     const GroupPlan old = plan(have_ws, false);
     if (old.ok && old.ws_bytes == 0) {    // fits as it is: unsplit, and lean if that can be
@@ -2938,13 +2962,8 @@ hipError_t group_entry(GroupFam fam, const void* kargs, int count, int out_dtype
     int span_begin[qg::kGroupMax + 1];
     hipError_t st = group_collect(fam, kargs, count, out_dtype, &g, span_begin);
     if (st != hipSuccess) return st;
-    const GroupPlan pl = group_plan(fam, g, ws != nullptr, aligned(ws, 256) ? ws_bytes : 0);
-    if (!pl.ok) return hipErrorInvalidValue;
-    if (ws && pl.ws_bytes) {
-        if (ws_bytes < pl.ws_bytes || !aligned(ws, 256)) return hipErrorInvalidValue;
-        for (int i = 0; i < g.spans; ++i)
-            if (overlaps(ws, pl.ws_bytes, g.span_p[i], g.span_b[i])) return hipErrorInvalidValue;
-    }
+    const GroupPlan pl = group_plan(fam, g, ws != nullptr, ws, ws_bytes);
+    if (!pl.ok || (ws && pl.ws_bytes && !group_holds(g, ws, ws_bytes, pl.ws_bytes))) return hipErrorInvalidValue;
     st = check_arch();
     if (st != hipSuccess) return st;
     const auto turn = workspace_turn(ws);
@@ -2988,7 +3007,7 @@ size_t group_workspace(GroupFam fam, const void* kargs, int count) {
     GroupCall g;
     int span_begin[qg::kGroupMax + 1];
     if (group_collect(fam, kargs, count, QGEMM_OUT_BF16, &g, span_begin) != hipSuccess) return 0;
-    const GroupPlan pl = group_plan(fam, g, true, SIZE_MAX);
+    const GroupPlan pl = group_plan(fam, g, true, nullptr, SIZE_MAX);
     return pl.ok ? pl.ws_bytes : 0;
 }
 

@@ -132,3 +132,56 @@ def test_launches_of_a_shared_workspace_stay_together(stub, plan):
     one = "noalloc(mx_kargs(2, 4, 7168, 32768, True))" if plan == "noalloc" else "bs(bs_kargs(2, 32, 1536, 7168))"
     name, call = SHARED[plan]
     assert _child(stub, SHARED_BODY % (call % 0, call % 1, one, name)) == ["0"]
+
+
+# shapes whose split ring plan (grouped: split plan) takes the place of one that needs no workspace
+KEPT = {
+    "mxfp8": "L.gemm_a8w8_mxfp8, L.gemm_a8w8_mxfp8_workspace_bytes, mx_kargs(0, 32, 2112, 8192)",
+    "mxfp4": "L.gemm_a4w4_mxfp4, L.gemm_a4w4_mxfp4_workspace_bytes, mx_kargs(0, 40, 4096, 16384, True)",
+    "bs": "L.gemm_a8w8_blockscale_bpreshuffle, L.gemm_a8w8_blockscale_bpreshuffle_workspace_bytes, "
+          "bs_kargs(0, 4, 2112, 16384)",
+    "bypass": "L.gemm_a8w8_blockscale_ldsbypass, L.gemm_a8w8_blockscale_ldsbypass_workspace_bytes, "
+              "bypass_kargs(0, 4, 2112, 16384)",
+}
+KEPT_BODY = """
+def bypass_kargs(at, m, n, k):
+    kg, p = k // 128, [far(5 * at + j) for j in range(5)]
+    return q.LdsBypassKargs(p[0], None, p[1], p[2], m, n, k, 1, k, 128, n, m * k, n * k, m * n, p[3], p[4],
+                            1 if m > 1 else m, kg, m * kg, (n + 127) // 128 * kg, (n + 15) // 16 * 16 * k)
+
+fn, query, a = %s
+need, ws = query(ctypes.byref(a)), far(100)
+b = a.ptr_b_pp if hasattr(a, "ptr_b_pp") else a.ptr_b
+assert need > 0
+
+def call(p, size):
+    st = fn(ctypes.byref(a), 1, P(p), size, None)
+    return st, q.last_launch().split("<")[0]
+
+st, plain = call(None, 0)
+assert st == 0 and plain != "ring_gemm", (st, plain)
+print(call(ws, need) == (0, "ring_gemm"))
+print(all(call(p, size) == (0, plain) for p, size in ((ws + 16, need), (a.ptr_c, need), (b, need), (ws, need - 1))))
+"""
+
+
+@pytest.mark.parametrize("entry", list(KEPT))
+def test_a_workspace_no_plan_can_use_is_no_error(stub, entry):
+    """Where the plan without the ring kernel needs no workspace, one that is
+    unaligned, on an operand or too small leaves the call to that plan."""
+    assert _child(stub, KEPT_BODY % KEPT[entry]) == ["True", "True"]
+
+
+GROUPED_BODY = """
+ks = (q.Kargs * 3)(*[bs_kargs(i, 32, n, k) for i, (n, k) in enumerate([(2112, 7168), (4096, 7168), (7168, 2048)])])
+fn, ws = L.gemm_a8w8_blockscale_bpreshuffle_grouped, far(100)
+need = L.gemm_a8w8_blockscale_bpreshuffle_grouped_workspace_bytes(ks, 3)
+assert need > 0
+for p, size in ((None, 0), (ws, need), (ws + 16, need), (ks[1].ptr_c, need), (ks[2].ptr_b, need), (ws, need - 1)):
+    print(fn(ks, 3, 1, 0, P(p), size, None))
+"""
+
+
+def test_grouped_workspace_no_plan_can_use_is_no_error(stub):
+    """The grouped entries alike: three problems that also run unsplit."""
+    assert _child(stub, GROUPED_BODY) == ["0"] * 6
