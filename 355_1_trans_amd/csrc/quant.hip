@@ -610,7 +610,8 @@ hipError_t launch_quant_rows(int fmt, int group, bool bf16in, bool shuffle, cons
     int lc = tall ? 5 : 7;
     while (!shuffle && lc > (group == 32 ? 2 : 4) && (4LL << lc) >= k) --lc;
     p.lc = lc;
-    p.ctiles = (k + (8 << lc) - 1) / (8 << lc);
+    // (k rounded up to a tile passes INT_MAX; the last unit's column, 2^31 - 8, does not)
+    p.ctiles = (int)((k + (8LL << lc) - 1) >> (lc + 3));
     const long long prow = shuffle ? (rows + 31LL) / 32 * 32 : rows;
     const long long passes = (prow + (256 >> lc) - 1) / (256 >> lc) * p.ctiles;
     const bool one = passes <= kQuantOnePass;

@@ -299,3 +299,16 @@ def test_device_quantized_operands_feed_the_gemms(qgemm, gpu):
     (ra8, rsa), (rb8, rsb) = O.quant_bs_act(a), O.quant_bs_wgt(b)
     y = qgemm.gemm_a8w8_bpreshuffle(qa8, qgemm.shuffle_b_kpanel(qb8), sa, sb, dtype=torch.float32)
     assert_close(O.gemm_bs_fp32(ra8, rb8, rsa, rsb), y.cpu().numpy(), "bs fp32")
+
+
+def test_longest_row(qgemm, gpu):
+    """One row of 2^31 - 128 elements: the codes and scales of the same
+    elements as rows of 128."""
+    k = 2 ** 31 - 128
+    x = torch.randn((k // 128, 128), generator=torch.Generator(gpu).manual_seed(3), device=gpu, dtype=torch.bfloat16)
+    for fn in (qgemm.quant_fp8_blockscale, lambda t: qgemm.quant_fp8_blockscale(t, scale_layout="km"),
+               qgemm.quant_mxfp8, qgemm.quant_mxfp4):
+        (q, s), (qr, sr) = fn(x.view(1, k)), fn(x)
+        assert q.shape[0] == 1 and torch.equal(q.view(torch.uint8).view(-1), qr.view(torch.uint8).view(-1))
+        assert torch.equal(s.reshape(-1), sr.reshape(-1))
+        del q, s, qr, sr

@@ -185,3 +185,24 @@ for p, size in ((None, 0), (ws, need), (ws + 16, need), (ks[1].ptr_c, need), (ks
 def test_grouped_workspace_no_plan_can_use_is_no_error(stub):
     """The grouped entries alike: three problems that also run unsplit."""
     assert _child(stub, GROUPED_BODY) == ["0"] * 6
+
+
+QUANT_BODY = """
+x, c, s = far(0), far(10), far(20)
+k, kg = (1 << 31) - 128, ((1 << 31) - 128) // 128
+for fn, args, tile in (
+        (L.qgemm_quant_fp8_blockscale_act, (c, k, s, kg, 1), 1024),
+        (L.qgemm_quant_fp8_blockscale_act, (c, k, s, 1, 8), 256),
+        (L.qgemm_quant_fp8_e8m0_act, (c, k, s, 1, 8), 256), (L.qgemm_quant_mxfp8, (c, k, s, 4 * kg, 0), 1024),
+        (L.qgemm_quant_mxfp4, (c, k // 2, s, 4 * kg, 0), 1024), (L.qgemm_quant_mxfp4, (c, k // 2, s, 4 * kg, 1), 256)):
+    stub.stub_reset(0)
+    st = fn(P(x), 1, 1, k, k, P(args[0]), args[1], P(args[2]), *args[3:], None)
+    # every tile of the row; the shuffled scales' tiles take 32 rows in one pass of four
+    print(st == 0 and stub.stub_count() == 1 and launches()[0][1] == (k + tile - 1) // tile)
+"""
+
+
+def test_quantizers_take_the_longest_row(stub):
+    """One row of 2^31 - 128 elements: the tile count is one past what int
+    arithmetic on the rounded-up K holds."""
+    assert _child(stub, QUANT_BODY) == ["True"] * 6
