@@ -276,6 +276,7 @@ struct QuantArgs {
     int kg8;                 // e8m0_shuffle: K/32 rounded up to 8
     int lc;                  // log2 of the tile's units of 8 columns
     int ctiles;              // tiles along K
+    unsigned grid_x;         // gridDim.x
 };
 
 // Row-wise group quantizer, GROUP elements per scale (32 for MX, 128 for
@@ -312,7 +313,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs p) {
     typedef typename std::conditional<FMT == 0, float, uint8_t>::type Scale;
     __shared__ Scale sc_tile[NSC];
     const int t = threadIdx.x, lc = p.lc;
-    const int rt = (int)(blockIdx.x / (unsigned)p.ctiles), ct = (int)(blockIdx.x - (unsigned)rt * (unsigned)p.ctiles);
+    const unsigned blk = blockIdx.y * p.grid_x + blockIdx.x;    // (past the last tile: every row is masked)
+    const int rt = (int)(blk / (unsigned)p.ctiles), ct = (int)(blk - (unsigned)rt * (unsigned)p.ctiles);
     const int rpp = 256 >> lc;                     // rows per pass
     const long long row0 = (long long)rt * (U * rpp);
     const int lr = t >> lc, lu = t & ((1 << lc) - 1), col = (ct << (lc + 3)) + 8 * lu;
@@ -577,6 +579,7 @@ __global__ __launch_bounds__(256) void e8m0_shuffle_blocks_kernel(const ShuffleA
 // Row passes of 256 threads up to which the row quantizer runs one per
 // workgroup: 2048 workgroups are one round of the chip at eight per CU.
 constexpr long long kQuantOnePass = 2048;
+constexpr long long kGridMaxX = 0xffffffffLL / 256;    // workgroups of 256
 
 unsigned grid_for(long long units) {
     const long long b = (units + 255) / 256;
@@ -618,7 +621,10 @@ hipError_t launch_quant_rows(int fmt, int group, bool bf16in, bool shuffle, cons
     const long long rpt = (256 >> lc) * (one ? 1 : 4);
     const long long blocks = (prow + rpt - 1) / rpt * p.ctiles;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    const unsigned grid = (unsigned)blocks;
+    // a grid dimension holds 2^32 threads at most: more tiles take a second one
+    const unsigned gy = (unsigned)((blocks + kGridMaxX - 1) / kGridMaxX);
+    p.grid_x = (unsigned)((blocks + gy - 1) / gy);
+    const dim3 grid(p.grid_x, gy);
 #define QG_QUANT(F, G, B, S)                                                                            \
     if (fmt == F && group == G && bf16in == B && shuffle == S) {                                        \
         if (one) quant_rows_kernel<F, G, B, S, 1><<<grid, 256, 0, st>>>(p);                             \

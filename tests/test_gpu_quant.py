@@ -312,3 +312,19 @@ def test_longest_row(qgemm, gpu):
         assert q.shape[0] == 1 and torch.equal(q.view(torch.uint8).view(-1), qr.view(torch.uint8).view(-1))
         assert torch.equal(s.reshape(-1), sr.reshape(-1))
         del q, s, qr, sr
+
+
+def test_more_tiles_than_one_grid_dimension(qgemm, gpu):
+    """Shuffled MXFP4 of 2^29 + 64 rows of 32: 2^24 + 2 workgroups.  The rows
+    at both ends have the bytes that they have alone."""
+    rows, part = 2 ** 29 + 64, 64
+    x = torch.zeros((rows, 32), device=gpu, dtype=torch.bfloat16)
+    ends = [torch.randn((part, 32), generator=torch.Generator(gpu).manual_seed(i), device=gpu, dtype=x.dtype)
+            for i in (0, 1)]
+    x[:part], x[-part:] = ends
+    q, e = qgemm.quant_mxfp4(x, shuffle=True)
+    del x
+    for i, (a, b) in enumerate(((q[:part], e[:part * 8]), (q[-part:], e[-part * 8:]))):
+        want = qgemm.quant_mxfp4(ends[i], shuffle=True)
+        assert torch.equal(a, want[0]) and torch.equal(b, want[1])
+    assert int(q[part:-part].max()) == 0 and int(e[part * 8:-part * 8].min()) == 127 == int(e[part * 8:-part * 8].max())

@@ -206,3 +206,19 @@ def test_quantizers_take_the_longest_row(stub):
     """One row of 2^31 - 128 elements: the tile count is one past what int
     arithmetic on the rounded-up K holds."""
     assert _child(stub, QUANT_BODY) == ["True"] * 6
+
+
+MANY_ROWS_BODY = """
+x, c, s, rows = far(0), far(10), far(20), (1 << 29) + 64    # K = 32, shuffled: 32 rows a workgroup
+for fn, row in ((L.qgemm_quant_mxfp8, 32), (L.qgemm_quant_mxfp4, 16)):
+    stub.stub_reset(0)
+    st = fn(P(x), 1, rows, 32, 32, P(c), row, P(s), 1, 1, None)
+    _, gx, gy, gz, threads, _ = launches()[0]
+    print(st == 0 and threads == 256 and gx * threads < 1 << 32 and rows // 32 <= gx * gy * gz < rows // 32 + gy)
+"""
+
+
+def test_quantizers_take_more_tiles_than_one_grid_dimension(stub):
+    """More than 2^24 workgroups of 256 threads: past what one dimension of a
+    grid may count."""
+    assert _child(stub, MANY_ROWS_BODY) == ["True"] * 2
