@@ -34,6 +34,7 @@ buffer per (device, stream); pass a tensor to supply your own, or
 import ctypes
 import importlib.machinery
 import importlib.util
+import warnings
 from functools import lru_cache
 from pathlib import Path
 
@@ -194,22 +195,32 @@ class _NoFast:
         return None
 
 
+_fast = None
+
+
 def fast():
     """The native form of the wrappers' plain calls (_fast.so, built with the
     library): ``gemm`` and ``quant`` return None for a call that the Python
     code has to check or make."""
-    return _fast_module() if LIB_PATH.exists() else _NoFast
+    return _fast or _load_fast()
 
 
-@lru_cache(None)
-def _fast_module():
+def _load_fast():
+    global _fast
     path = _PKG / "_fast.so"
-    if not path.exists():
+    if not LIB_PATH.exists():    # the Python code's lib() says so
         return _NoFast
-    loader = importlib.machinery.ExtensionFileLoader("_fast", str(path))
-    mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_fast", path, loader=loader))
-    loader.exec_module(mod)
-    mod.bind(*[ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _FAST_CALLS])
+    mod = _NoFast
+    if path.exists():
+        loader = importlib.machinery.ExtensionFileLoader("_fast", str(path))
+        try:
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_fast", path, loader=loader))
+            loader.exec_module(mod)
+            mod.bind(*[ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _FAST_CALLS])
+        except (ImportError, TypeError) as e:    # built for another torch, Python or library
+            warnings.warn(f"{path} cannot be used, calls go through Python: {e}")
+            mod = _NoFast
+    _fast = mod
     return mod
 
 

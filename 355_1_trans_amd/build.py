@@ -4,11 +4,13 @@ Every ``csrc/*.hip`` file is compiled to an object under ``_build/`` (in
 parallel) and linked into ``libqgemm.so`` next to this file.  All HIP code is
 compiled with packed-FP32 instruction generation disabled.  ``csrc/host/fast.cpp``
 (host code against torch's headers: the Python wrappers' plain calls) becomes
-``_fast.so``.
+``_fast.so``; where it cannot be built (no torch, no g++) a warning says so, and
+the wrappers make those calls in Python.
 """
 import os
 import subprocess
 import sys
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -42,6 +44,7 @@ def _compile(src: Path) -> Path:
 
 
 def _build_fast() -> None:
+    FAST.unlink(missing_ok=True)    # never one of an older library
     import sysconfig
 
     import torch
@@ -67,13 +70,14 @@ def build(jobs: int = 8, verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=max(1, min(jobs, len(sources)))) as ex:
         fast = ex.submit(_build_fast)
         objs = list(ex.map(_compile, sources))
-        fast.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
+    if fast.exception():
+        warnings.warn(f"{FAST.name} was not built, calls go through Python: {fast.exception()}")
     if verbose:
         print(f"built {LIB}")
     return LIB

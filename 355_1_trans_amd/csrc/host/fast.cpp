@@ -5,8 +5,8 @@
 // wrapper took 14.5 us of host time: two 1.7 us allocations, 1.8 us for the
 // stream object, 1.3 us for the device guard, 4-4.6 us in the launch itself,
 // the rest checks, ctypes conversions and record_stream calls.  Here the same
-// steps take 6.2 us, most of it the launch: one token through a 7168 -> 2112
-// block-scale layer (quantizer and GEMM) 26 -> 13.6 us per pass.
+// steps take 5.0-5.5 us, most of it the launch: one token through a 7168 ->
+// 2112 block-scale layer (quantizer and GEMM) 26 -> 12.1 us per pass.
 //
 // Every function returns None for a call that is not plain -- another
 // tensor type than torch.Tensor, a shape, stride, type or device the entry
