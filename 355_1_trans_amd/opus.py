@@ -31,8 +31,9 @@ from . import Kargs, _Address, _check, _out_code, _record, _require_gpu, _stream
 CONFIGS = Path(__file__).resolve().parent / "configs"
 
 KID_AUTO, KID_TILE256, KID_MID, KID_SKINNY, KID_DECODE, KID_BURST = range(6)
+KID_RING = 11    # ids 6 - 10 are the MX entries' own
 KID_NAMES = {KID_AUTO: "auto", KID_TILE256: "tile256", KID_MID: "mid128", KID_SKINNY: "skinny",
-             KID_DECODE: "decode", KID_BURST: "burst"}
+             KID_DECODE: "decode", KID_BURST: "burst", KID_RING: "ring"}
 LAYOUTS = {"nt": 0, "nn": 1, "tt": 2, "tn": 3}
 
 _WS = {}

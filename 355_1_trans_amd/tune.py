@@ -183,7 +183,7 @@ def tune_shape(q, m, n, k, variant, kids, dev, stream):
 
 
 MX_KIDS = {0: "auto", 1: "tile256", 2: "mid128", 3: "skinny", 4: "decode", 5: "burst", 6: "stream", 7: "band",
-           8: "quad", 9: "runs", 10: "slice"}
+           8: "quad", 9: "runs", 10: "slice", 11: "ring"}
 
 
 def tune_shape_mx(q, m, n, k, fp4, kids, dev, stream):
@@ -298,6 +298,7 @@ def main():
     props = torch.cuda.get_device_properties(dev)
     gfx = getattr(props, "gcnArchName", "gfx950").split(":")[0]
     cu_num = props.multi_processor_count
+    # the table's ids; the ring kernel (11) comes into it by AUTO's rule, `--kids` times it by itself
     kids = [int(x) for x in (args.kids or "0,1,2,3,4,5").split(",")]
     if args.grid:
         shapes = _grid(args.grid)

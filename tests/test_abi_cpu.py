@@ -492,3 +492,31 @@ def test_slice_kernel_id_contract(qgemm):
     assert L.gemm_a4w4_mxfp4_kid(ctypes.byref(a), 1, kid, None, 0, None) == HIP_INVALID_VALUE
     a = _far_kargs(qgemm, 32, 7168, 16384, fp4=True)
     assert L.gemm_a4w4_mxfp4_kid(ctypes.byref(a), 1, kid, None, 0, None) == HIP_INVALID_VALUE   # split needs ws
+
+
+def test_ring_kernel_id_contract(qgemm):
+    """QGEMM_KID_RING (11): M <= 64 in every family; a split sizes its
+    workspace as counters + fp32 planes and needs it aligned; without one the
+    id runs unsplit; other shapes answer 0 / hipErrorInvalidValue, dimensions
+    near INT_MAX included."""
+    L = qgemm.lib()
+    kid, big = 11, (1 << 31) - 1
+    q = lambda a: L.gemm_a8w8_mxfp8_kid_workspace_bytes(ctypes.byref(a), kid)
+    assert q(_far_kargs(qgemm, 65, 7168, 16384)) == 0                            # M > 64
+    assert q(_far_kargs(qgemm, 64, 16384, 2048)) == 0                            # tiles for every CU: unsplit
+    for m, n, k in ((1, 512, 16384), (32, 1536, 7168), (64, 2112, 8192)):       # split
+        a = _far_kargs(qgemm, m, n, k)
+        need, ws = q(a), (1 << 44) + (7 << 38)
+        assert need > 2048 and (need - 2048) % (m * n * 4) == 0, (m, n, k, need)
+        call = lambda p, size: L.gemm_a8w8_mxfp8_kid(ctypes.byref(a), 1, kid, p, size, None)
+        for p, size in ((ws, need - 1), (ws + 16, need), (a.ptr_c, need)):
+            assert call(p, size) == HIP_INVALID_VALUE, (m, n, k)
+        if not torch.cuda.is_available():
+            assert call(ws, need) != HIP_INVALID_VALUE and call(None, 0) != HIP_INVALID_VALUE
+    a = _far_kargs(qgemm, 65, 7168, 16384)
+    assert L.gemm_a8w8_mxfp8_kid(ctypes.byref(a), 1, kid, None, 0, None) == HIP_INVALID_VALUE
+    for m, n in ((1, big), (64, big - 15), (big, 1)):
+        a = _kargs(qgemm, m=m, n=n)
+        for query in ("gemm_a8w8_mxfp8", "gemm_a4w4_mxfp4", "gemm_a8w8_blockscale_bpreshuffle"):
+            getattr(L, query + "_kid_workspace_bytes")(ctypes.byref(a), kid)
+        assert L.gemm_a8w8_mxfp8_kid(ctypes.byref(a), 1, kid, None, 0, None) == HIP_INVALID_VALUE

@@ -63,3 +63,15 @@ def test_tuner_mx_reference_dequant():
     assert np.array_equal(got8, O.e4m3_decode(fp8) * np.repeat(O.e8m0_decode(e2), 32, axis=1))
     assert tune._grid("24576,32768:1536:32,64") == [(32, 24576, 1536), (64, 24576, 1536), (32, 32768, 1536),
                                                   (64, 32768, 1536)]
+
+
+def test_every_kernel_id_has_a_name(qgemm):
+    """The tuner and the aiter-facing module name every QGEMM_KID_* their entries take."""
+    import importlib
+    import re
+    tune = importlib.import_module("355_1_trans_amd.tune")
+    header = (ROOT / "include" / "qgemm.h").read_text()
+    ids = {name: int(v) for name, v in re.findall(r"#define QGEMM_KID_(\w+)\s+(\d+)", header)}
+    assert set(tune.MX_KIDS) == set(ids.values())
+    assert {"AUTO", "TILE256", "MID", "SKINNY", "DECODE", "BURST", "RING"} <= set(ids)
+    assert set(qgemm.opus.KID_NAMES) == {ids[n] for n in ("AUTO", "TILE256", "MID", "SKINNY", "DECODE", "BURST", "RING")}
