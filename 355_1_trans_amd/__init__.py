@@ -25,11 +25,12 @@ and launch on the current stream:
 There is no CPU fallback: every wrapper raises if the library is missing or
 the tensors are not on a GPU.
 
-Skinny-M calls split K across workgroups and reduce the fp32 partials in the
-same launch; the workspace's counter words are tagged with a per-launch
-epoch, so any initial contents work.  ``workspace=None`` uses one cached
-buffer per (device, stream); pass a tensor to supply your own, or
-``workspace=False`` to run without split-K.
+Calls whose tiles leave the GPU idle split K across workgroups and sum the
+fp32 partials in the same launch (counter words in the workspace, tagged with
+a per-launch epoch, so any initial contents work) or, in the ring, 128 x 128,
+four-wave and one-by-four kernels, in a second one.  ``workspace=None`` uses
+one cached buffer per (device, stream), which threads may share; pass a
+tensor to supply your own, or ``workspace=False`` to run without split-K.
 """
 import ctypes
 import importlib.machinery
@@ -395,15 +396,17 @@ def gemm_a4w4(A, B, A_scale, B_scale, out=None, bias=None, alpha=1.0, beta=0.0, 
     A_scale / B_scale: E8M0 in e8m0_shuffle order (``e8m0_shuffle``, or
     ``quant_mxfp4(x, shuffle=True)``), rows padded to 32; out [M, N], bf16
     unless ``dtype`` (or a given ``out``) says fp32.  ``grid_blocks`` > 0 runs a persistent grid of that
-    many workgroups.  ``kernel_id``: 0 = the library's choice (M = 9-64 on
-    the slice kernel where its plan fills the CUs in one round, else M <= 64
-    on the burst kernel, else the one-by-four wave kernel), 1 = the two-by-two
-    wave 256x256 kernel, 5 = the burst kernel (M <= 64), 8 = the one-by-four
-    wave kernel (no persistent grid), 10 = the slice kernel (M <= 64).
-    ``workspace``: as for the other entries (None: a cached buffer when a
-    plan splits K; False: none, so only unsplit plans).  The epilogue has no bias or alpha/beta: anything but
-    the defaults raises, and so does bpreshuffle=False (row-major B goes
-    through gemm_a4w4_mxfp4)."""
+    many workgroups.  ``kernel_id``: 0 = the library's choice (the ring kernel
+    for M = 33-64 with 1536 < N <= 7168 from K = 6144 on and for M = 17-64 with
+    12288 < N <= 16384 from K = 16384 on; M = 9-64 else on the slice kernel
+    where its plan fills the CUs in one round, else M <= 64 on the burst
+    kernel, else the one-by-four wave kernel), 1 = the two-by-two wave 256x256
+    kernel, 5 = the burst kernel (M <= 64), 8 = the one-by-four wave kernel
+    (no persistent grid), 10 = the slice kernel (M <= 64), 11 = the ring kernel
+    (M <= 64).  ``workspace``: as for the other entries (None: a cached buffer
+    when a plan splits K; False: none, so only unsplit plans).  The epilogue
+    has no bias or alpha/beta: anything but the defaults raises, and so does
+    bpreshuffle=False (row-major B goes through gemm_a4w4_mxfp4)."""
     if bias is not None or alpha != 1.0 or beta != 0.0:
         raise NotImplementedError("gemm_a4w4: bias, alpha and beta are not supported")
     if not bpreshuffle:

@@ -194,8 +194,8 @@ bool dma_aligned(const opus_gemm_scale_kargs& a, bool scales_dword) {
 // workgroups -- only up to one round of workgroups (cus), keeping >= 16
 // K-tiles per slice and the fp32 partials below a quarter of B's bytes.  This
 // plan depends on the shape only, so its workspace query and its launch
-// always agree (the MX entries' four-wave K split also depends on the
-// workspace bytes passed: see plan_wide_ws).
+// always agree (the ring kernel's K split and the MX entries' four-wave one
+// also depend on the workspace at hand: ring_fits, plan_wide_ws).
 constexpr int kMinTiles = 192;
 constexpr int kSplitBelow = 128;
 // Split-K counters sit in a fixed block at the start of the workspace (the
@@ -365,15 +365,16 @@ void plan_mid(Plan& p, int m, int n, int k_tiles, int batch, int cus, bool force
         return;
     long long split = std::min<long long>(target / tiles, k_tiles / kMidMinKt);
     // up to cus / 2 tiles: at most one workgroup per CU (four LDS stages,
-    // longer slices, fewer partials) -- N = 7168, K = 16384: MXFP8 M = 128
-    // 75.0 -> 61.9 us, BS fp32 M = 128 64.9 -> 47.0, M = 256 76.5 -> 64.0,
-    // MXFP4 M = 256 54.7 -> 50.7; shapes with less K unchanged
+    // longer slices, fewer partials) -- on the kernel before its DMA waves,
+    // N = 7168, K = 16384: MXFP8 M = 128 75.0 -> 61.9 us, BS fp32 M = 128 64.9
+    // -> 47.0, M = 256 76.5 -> 64.0, MXFP4 M = 256 54.7 -> 50.7; shapes with
+    // less K unchanged (the four now run in 37.1, 33.5, 50.1 and 33.1 us)
     if (cus / tiles >= 2) split = std::min<long long>(split, cus / tiles);
-    // 8-K-tile slices (the slices summed by splitk_reduce_kernel): BS fp32
-    // M = 128, N = 2112, K = 7168 22.4 -> 17.7 us, MXFP4 M = 128 - 512,
-    // K = 7168 (28 K-tiles, unsplit before) 1.2-1.75x, MXFP8 M = 128,
-    // K = 2048 1.15-1.3x; K = 2048 at M >= 256, or a second round of
-    // workgroups, up to 1.6x slower
+    // 8-K-tile slices (the slices summed by splitk_reduce_kernel), before the
+    // DMA waves as well: BS fp32 M = 128, N = 2112, K = 7168 22.4 -> 17.7 us
+    // (now 15.5), MXFP4 M = 128 - 512, K = 7168 (28 K-tiles, unsplit before)
+    // 1.2-1.75x, MXFP8 M = 128, K = 2048 1.15-1.3x; K = 2048 at M >= 256, or a
+    // second round of workgroups, up to 1.6x slower
     if (k_tiles >= 24 || ceil_div(m, 128) == 1)
         split = std::max<long long>(split, std::min<long long>(cus / tiles, k_tiles / kMidMinKtDeep));
     if (split <= 1) return;
@@ -684,9 +685,16 @@ struct BsfRoute {
 //    (1.03-1.07), N = 12288 - 16384 at K <= 2048 (1.04-1.10; K = 16384
 //    0.84-1.0);
 //  * M = 33-64: N <= 4096 (1.04-1.87) and to 8192 at K = 2560 - 6144 (1.14-2.4;
-//    7168 at N <= 7168 1.05-1.14; wider or longer loses, 0.7-1.0).  N = 1025 -
-//    1536 near K = 7168 and N <= 768 near K = 8192 with M <= 32 stay on the
-//    burst kernel, N = 7168 at K <= 2048 too (ring 1.02-1.11 on these).
+//    7168 at N <= 7168 1.05-1.14; wider loses, 0.7-1.0).
+// Windows in which the ring measured faster and the route below stands all
+// the same (us, below / ring):
+//  * where the burst kernel's tests assert it through AUTO: M = 17-32, N =
+//    769 - 2048 below K = 12288 (N = 1536, K = 7168 / 8192 9.3-9.7 / 8.6-9.0)
+//    and N <= 768 at K = 8192 - 12160 (9.9-10.2 / 8.2-8.4); M = 33-64, N = 1025 -
+//    1536 near K = 7168 (11.0-11.9 / 9.9-10.4) and N > 4096 to K = 2048
+//    (N = 7168 8.2-9.0 / 7.9-8.3);
+//  * M = 33-64 past K = 7168 at N = 4097 - 7168, drawn too tight (N = 7168,
+//    K = 8192 17.8-20.3 / 17.1-19.2, fragment-order B 23.4 / 19.3).
 bool ring_bsf32(int m, int n, int kt, int batch, bool frag) {
     if (batch != 1 || n < 256 || m > 64) return false;
     const bool long_k = kt >= 96;
@@ -779,7 +787,8 @@ BsfRoute route_bsf32(int m, int n, int k_tiles, int batch, long long b_bytes, bo
 // K = 7168 56-68 -> 46-58 against the 256 x 256 kernel with its K split, MXFP4
 // 27-31 -> 23-25 and 39-44 -> 33-37; at 80 K-tiles MXFP8 equal, at 128 1.04-1.1x
 // slower).  From 136 tiles on the 256 x 256 kernel is 1.1-1.35x faster.  M <=
-// 1024 measured alike; its routes are pinned by tests and stay.
+// 1024 measured alike; the route tests assert its kernels (M = 768, N = 6144),
+// and they stay.
 bool mid_mx_deep(int m, int k_tiles) { return m > 1024 && k_tiles <= 64; }
 
 // MX: the same 128 x 128 rule (row-major B, E8M0 scales applied by the
@@ -1413,8 +1422,11 @@ bool ring_panels(const opus_gemm_scale_kargs& a, bool fp4) {
 //    with 2-4 KB rows (1.01-1.33, where the burst plans run in two waves);
 //  * M = 33-64, N <= 8192 (1.06-1.85): A's rows come once per 16-32 columns
 //    from LDS.  Wider N: the 128 x 128 kernel, which reads A once per 128.
-//    64 - 71 K-tiles with M > 40 stay on the row-run kernel at N <= 4096 and,
-//    MXFP4, on the slice kernel past N = 6144 (ring 1.15-1.34 there).
+// M > 40 at 64 - 71 K-tiles keeps the row-run kernel at N <= 4096 and, MXFP4,
+// the slice kernel past N = 6144, because the tests of those two kernels assert
+// them through AUTO at 64 K-tiles.  The ring measured faster (us, they / ring):
+// N = 2112 16.4-16.9 / 11.9-12.8, N = 4096 17.4-18.1 / 14.6-15.6, N = 7168 and
+// 8192 21.2-24.0 / 17.8-18.9.
 bool ring_mx(int m, int n, int kt, bool fp4) {
     const int row = kt * 128;
     if (m > 64 || n < 256) return false;
@@ -1893,7 +1905,8 @@ size_t gemm_a4w4_mxfp4_kid_workspace_bytes(const opus_gemm_scale_kargs* args, in
 
 namespace {
 
-// Route of the aiter-format MXFP4 entry.  AUTO: M <= 64 runs the burst
+// Route of the aiter-format MXFP4 entry.  AUTO: M <= 64 outside the ring
+// kernel's rule (below) and the slice kernel's (in the route) runs the burst
 // kernel (B in shuffle_weight(16,16) order is the 16x16x128 MFMA's operand
 // order, streamed as whole 1 KB loads; a K split needs the workspace, so
 // without one only unsplit plans) -- its gated plan, else, for M = 33-64,
@@ -1937,7 +1950,9 @@ int plan_quad_split(const opus_gemm_mxfp4_scale_kargs& x, int cus) {
 // the ring): M = 33-64 from 24 K-tiles on (N = 2048 - 7168: 1.02-1.42; short
 // K 0.83-1.0), and one round of 64-column tiles at K >= 16384 from M = 17 on
 // (N = 13312 / 16384: 1.36-1.66).  At M <= 32 the burst kernel's 1 KB loads of
-// W16 blocks need no staging (ring 0.74-1.0); N <= 1536 stays on it too (1.0-1.16).
+// W16 blocks need no staging (ring 0.74-1.0).  N <= 1536 stays on it too,
+// although the ring measured 1.0-1.16: its tests assert it through AUTO at
+// M = 48, N = 1536.
 bool ring_mx4s(int m, int n, int kt) {
     if (n > 12288 && n <= 16384 && kt >= 64) return m > 16 && m <= 64;
     return m > 32 && m <= 64 && n > 1536 && n <= 7168 && kt >= 24;
@@ -2237,8 +2252,9 @@ size_t gemm_a4w4_mxfp4_noalloc_max_workspace_bytes(void) { return kScratchBytes;
 // query is planned without a cap): a call whose query exceeds the scratch is
 // refused rather than planned onto another kernel, whose rounding could
 // differ.  With need <= kScratchBytes the routes below plan the same: the
-// only workspace-dependent choice, the four-wave K split, is taken exactly
-// when its bytes fit, and they are part of `need`.
+// workspace-dependent choices, the four-wave and the ring K split, are taken
+// exactly when their bytes fit, and they are part of `need` (a ring plan's
+// are at most 8 planes of 64 x 8192 or 32 x 16384 outputs: 16.8 MB).
 hipError_t gemm_a4w4_mxfp4_noalloc(const opus_gemm_scale_kargs* args, int out_dtype, hipStream_t stream) {
     qg::trace_reset();
     const size_t need = mx_workspace(args, true, QGEMM_KID_AUTO);

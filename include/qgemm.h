@@ -149,10 +149,13 @@ size_t gemm_a8w8_blockscale_layout_workspace_bytes(const opus_gemm_scale_kargs* 
  * need no clearing (a completed call leaves them zero).  Calls that share a
  * workspace must be on one stream; they may come from several threads (a
  * call's launches -- some plans sum partial planes in a second one -- are
- * queued together, whatever other threads queue).  The MX entries' plan, and so
- * the rounding of their last bits, also depends on workspace_bytes: the
- * four-wave kernel's K split is taken only when its planes fit (a workspace
- * of at least the scale-panel bytes but less than the query runs unsplit). */
+ * queued together, whatever other threads queue).  The plan, and so the
+ * rounding of the last bits, also depends on the workspace at hand: with
+ * M <= 64 every AUTO entry takes the ring kernel's K split only where its
+ * planes can go into the workspace (else the plan without the ring kernel,
+ * which may need less or none), and the MX entries take the four-wave
+ * kernel's K split only where its planes fit (a workspace of at least the
+ * scale-panel bytes but less than the query runs unsplit). */
 hipError_t gemm_a8w8_blockscale_bpreshuffle(const opus_gemm_kargs* args, int out_dtype, void* workspace,
                                      size_t workspace_bytes, hipStream_t stream);
 size_t gemm_a8w8_blockscale_bpreshuffle_workspace_bytes(const opus_gemm_kargs* args);
@@ -293,11 +296,11 @@ hipError_t gemm_a4w4_mxfp4_bpreshuffle(const opus_gemm_mxfp4_scale_kargs* args, 
  * that takes grid_blocks > 0), QGEMM_KID_QUAD (one-by-four waves, B straight
  * from memory into registers), QGEMM_KID_BURST (M <= 64), QGEMM_KID_SLICE
  * (M <= 64: A's K slice in LDS, B's W16 fragments straight into registers) or
- * QGEMM_KID_RING (M <= 64: through an LDS ring filled by DMA waves); other ids, and shapes a forced id cannot take, are rejected.  The
- * workspace (size from the query below, 256-byte aligned, any contents)
- * carries a burst or slice plan's split-K counters and fp32 partials (a ring
- * plan's partials); the
- * plain entry above runs without one. */
+ * QGEMM_KID_RING (M <= 64: through an LDS ring filled by DMA waves); other
+ * ids, and shapes a forced id cannot take, are rejected.  The workspace (size
+ * from the query below, 256-byte aligned, any contents) carries a burst or
+ * slice plan's split-K counters and fp32 partials, a ring plan's and a split
+ * QUAD plan's partials; the plain entry above runs without one. */
 hipError_t gemm_a4w4_mxfp4_bpreshuffle_kid(const opus_gemm_mxfp4_scale_kargs* args, int out_dtype, int kernel_id,
                                            void* workspace, size_t workspace_bytes, hipStream_t stream);
 size_t gemm_a4w4_mxfp4_bpreshuffle_kid_workspace_bytes(const opus_gemm_mxfp4_scale_kargs* args, int kernel_id);
