@@ -447,7 +447,7 @@ def gemm_a8w8_bpreshuffle(A, B_kpanel, A_scale, B_scale, dtype=torch.bfloat16, o
     """Block-scale FP8 with fp32 scales.
 
     A [M,K] e4m3; B_kpanel [K/128, N, 128] e4m3 (shuffle_b_kpanel of B [N,K]);
-    A_scale fp32 [M,K/128] (row-major, BASELINE) or a [M,K/128] view with
+    A_scale fp32 [M,K/128] (row-major) or a [M,K/128] view with
     strides (1, M) (the reference's column-major [K/128][M]); B_scale fp32
     [ceil(N/128), K/128]."""
     if out is None and workspace is None:

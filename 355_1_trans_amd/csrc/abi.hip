@@ -1389,7 +1389,7 @@ void plan_wide_ws(MxRoute& r, const opus_gemm_scale_kargs& a, bool fp4, int cus,
 // (graph-replayed, MXFP4 / MXFP8 us): short K gains 1.1-1.5x over the skinny
 // kernel (fp4 M = 32: N = 24576, K = 1536 12.4 -> 9.4; N = 7168, K = 2048
 // 8.1 -> 5.6; fp8 M = 16, N = 24576, K = 1536 15.6 -> 10.7), long K loses
-// (fp4 configs[4] K = 16384, M = 16 / 32: 15.8 / 19.2 on the skinny kernel,
+// (fp4 N = 7168, K = 16384, M = 16 / 32: 15.8 / 19.2 on the skinny kernel,
 // 17.7 / 29.2 as a burst); M <= 8 stays on the row-streaming kernel, whose
 // contiguous row runs 16-row fragments cannot match (M = 1: 12.8 vs 17.5),
 // up to N = kStreamBurstN: past it the burst kernel's many short workgroups
@@ -1483,8 +1483,8 @@ MxRoute route_mx(const opus_gemm_scale_kargs& a, bool fp4, int kid, const Worksp
                 // 32-row band plans with long K slices (>= 12 K-tiles) over
                 // 7/10 or more of the CUs, where the slice kernel would split
                 // K: 128 columns of B per workgroup read once, with A's slice
-                // in LDS (graph-replayed, two boxes: MXFP4 configs[4] M = 32
-                // 16.7-18.2 us against 18.9-19.8 for the slice kernel and
+                // in LDS (graph-replayed, two boxes: MXFP4 M = 32, N = 7168,
+                // K = 16384 16.7-18.2 us against 18.9-19.8 for the slice kernel and
                 // 18.6-20.5 for the skinny one; M = 24 / 32, N = 4096-8192,
                 // K = 8192 / 16384, both formats: 8-20% faster than the
                 // slice kernel; unsplit slice plans, N = 12288-16384, keep
@@ -2719,7 +2719,7 @@ const char* qgemm_last_launch(void) { return qg::g_trace_str(); }
 // split-K reduce (R/opus_gemm_splitk_and_interface_refactor.md:41-45) and
 // the persistent tile walk of MX4/MULTITILE_DESIGN.md:78: a narrow-N decode
 // GEMM alone fills a fraction of the CUs and pays a launch of its own
-// (configs[2] M <= 64 at N = 2112-7168 run at 0.13-0.45 of HBM one by one).
+// (fp32 scales, M <= 64, N = 2112-7168 run at 0.13-0.45 of HBM one by one).
 namespace {
 
 struct GroupProblem {
@@ -2779,8 +2779,8 @@ GroupPlan plan_grouped(const GroupProblem* p, int count, bool mx, bool frag, int
     }
     const int mb = mmax <= 16 ? 1 : (mmax <= 32 ? 2 : 4);
     // 16 waves first: on a tie (the same items and bytes) the plan that puts
-    // twice the waves' loads in flight per item wins -- configs[2]'s decode
-    // trio, fp32 block scales, M = 1 / 16: 18.3 / 21.1 us with 8 waves x 8
+    // twice the waves' loads in flight per item wins -- the decode trio
+    // (N, K) = (2112, 7168), (4096, 7168), (7168, 2048), fp32 scales, M = 1 / 16: 18.3 / 21.1 us with 8 waves x 8
     // K-tiles, 17.5 / 19.2 us with 16 x 4
     for (int nb : {2, 1}) {
         if (lean && !mx && mb == 2 && nb == 1 && best.ok) {

@@ -169,8 +169,8 @@ __global__ __launch_bounds__(kBandWaves * 64, 1) void band_gemm_kernel(const Ban
             boff[j][h] = min(nw + j * 16 + R, N - 1) * LDB + c * 16;
         }
     // B is read once: non-temporal DMAs (one box, graph-replayed from HBM:
-    // configs[4] MXFP4 M = 32 17.8 -> 16.5 us, MXFP8 M = 32, N = 7168,
-    // K = 8192 17.1 -> 15.9, every band plan measured 4-8% faster)
+    // MXFP4 M = 32, N = 7168, K = 16384 17.8 -> 16.5 us, MXFP8 K = 8192
+    // 17.1 -> 15.9, every band plan measured 4-8% faster)
     auto load_b = [&](auto sc, int t) __attribute__((always_inline)) {
         const auto rB = rsrc(B, t < nk);    // past the slice: zeros, no memory read
         QG_LDS uint8_t* dst = ring(sc) + w * SLOT;

@@ -6,7 +6,7 @@
 // block's K-tile is the two 1 KB operands of the 16x16x128 MFMA) and both
 // scale tensors in e8m0_shuffle order.
 //
-// A decode GEMM streams B once; at configs[0] size (11 MB) the whole launch
+// A decode GEMM streams B once; at N = 1536, K = 7168 (11 MB) the whole launch
 // lasts a few microseconds, so what bounds it is how many bytes are in flight
 // at once, not a steady-state rate.  Measured on MI355X (graph-replayed
 // launches over rotating copies of an 11 MB operand): a launch that issues

@@ -93,8 +93,8 @@ __device__ __forceinline__ float load_partial1(__amdgpu_buffer_rsrc_t r, int ele
 // not waited for.  A word above the tag (a wrapped epoch, garbage) keeps its
 // value and the arrivals claim it by compare-and-swap instead.  Without the
 // claim every slice of a tile arriving close together found an untagged word
-// and went through the compare-and-swap loop: configs[0]'s five slices per
-// tile measured 13.6 us a launch against 9.1 us.
+// and went through the compare-and-swap loop: the five slices
+// per tile of M = 32, N = 1536, K = 7168 measured 13.6 us a launch against 9.1 us.
 __device__ __forceinline__ void split_claim(unsigned* ctr, unsigned epoch) {
     __hip_atomic_fetch_max(ctr, epoch << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -1,7 +1,7 @@
 // Slice decode GEMM for gfx950: MXFP8 / MXFP4 with row-major B, M <= 64.
 //
 // What bounds a decode GEMM's loads on MI355X (copy-only replays, 224
-// workgroups, 16 B per lane, configs[4]'s 7168 x 8 KB B):
+// workgroups, 16 B per lane, a 7168 x 8 KB B: MXFP4, K = 16384):
 //  * B straight from HBM in MFMA-fragment order (16 rows x 64 B per load)
 //    streams 5.3 TB/s when each wave walks one 16-row block over a contiguous
 //    2 KB of K (whether 8 or 32 loads are in flight), but 3.7 TB/s when each
@@ -23,7 +23,7 @@
 //    64-127 of 16 rows) go straight into registers, D K-tiles ahead, and meet
 //    A's fragments read from LDS -- B never passes through LDS and no wave
 //    waits for another inside the K loop; row-major B loads with the default
-//    cache policy (the non-temporal one ran configs[4] M = 1-64 10-15%
+//    cache policy (the non-temporal one ran that B at M = 1-64 10-15%
 //    slower), W16 B non-temporal;
 //  * the KQ waves of a block add their tiles in K order through LDS; a K
 //    split over workgroups uses the epoch-tagged counters and device-coherent
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kSliceWaves * 64, 1) void slice_gemm_kernel(const R
     const auto rSW = rsrc(SFB + (long long)(blk16 >> 1) * SFB_SN, nk * 256, kt_w * 256, W16 && (blk16 >> 1) < rows32b);
     const int b_off = W16 ? L * 16 : min(n0 + 16 * bw + l16, N - 1) * LDB + q * 16;
     constexpr int B_KT = W16 ? 2048 : BKB, B_HI = W16 ? 1024 : 64;
-    // cache policy of the B loads: non-temporal for W16 (aiter configs[4]
+    // cache policy of the B loads: non-temporal for W16 (N = 7168, K = 16384,
     // M = 32 / 64 18.4 / 22.1 -> 16.5 / 20.5 us with the rotated walk), the
     // default for row-major B (non-temporal 5-8% slower there)
     constexpr int B_AUX = W16 ? 2 : 0;
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kSliceWaves * 64, 1) void slice_gemm_kernel(const R
     // rotation every wave of the grid reads the same 2 KB offset of a 32 KB
     // K window at the same step, and with W16's contiguous 2 KB K-tiles those
     // reads crowd into few HBM channels: rotating by wave, K part and tile
-    // (weights replayed from HBM, one box: W16 configs[4] M = 16 / 32 / 48 /
+    // (weights replayed from HBM, one box: W16, that B, M = 16 / 32 / 48 /
     // 64 14.0 / 19.2 / 24.2 / 26.3 -> 13.8 / 18.2 / 20.3 / 22.0 us; row-major
     // 64-row plans 2.8-3.2% faster, its 16-row plans 2% slower, so those keep
     // the plain walk)

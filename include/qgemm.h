@@ -140,7 +140,7 @@ size_t gemm_a8w8_blockscale_layout_workspace_bytes(const opus_gemm_scale_kargs* 
  * K-panel layout [K/128][N][128] (stride_b = 128, BPS host.cc:92-111,263);
  * SFB fp32 [ceil(N/128)][K/128] (stride_sfb = K/128). SFA fp32 is either
  * the reference's column-major [K/128][M] (stride_sfa = M, BPS host.cc:270)
- * or BASELINE's row-major [M][K/128] (stride_sfa = 1). C bf16/fp32 [M,N].
+ * or row-major [M][K/128] (stride_sfa = 1). C bf16/fp32 [M,N].
  * Any M >= 1, N >= 1 (tails are masked), K a multiple of 128.
  * `workspace` (fp32 split-K partials) may be NULL; then no split-K is used.
  * Split-K workspace (every entry with a *_workspace_bytes query): at least
@@ -396,11 +396,11 @@ int qgemm_pack_b_ldsbypass(const uint8_t* b_raw, uint8_t* b_pp, int n, int k);
 /* Source: fp32 (in_dtype QGEMM_IN_FP32) or bf16 (QGEMM_IN_BF16) rows of K
  * elements, row pitch ldx >= K a multiple of 4 elements, base aligned to 16
  * (fp32) or 8 (bf16) bytes.  Codes are round-to-nearest-even, saturating,
- * bit-identical to the host recipes of BASELINE.json's configs.  Outputs
+ * bit-identical to the host recipes (scale = amax / 448 per block, or E8M0
+ * 2^ceil(log2(amax / qmax)) with qmax 448 or 6).  Outputs
  * must not overlap the source or each other.  The reference quantizes with
  * aiter (not in the container; its MXFP4 path is quant(..., shuffle=True),
- * MX4/candidate_m9/README.md:6-12), so these replace that step; the recipes
- * themselves are the ones BASELINE.json configs[0-4] state. */
+ * MX4/candidate_m9/README.md:6-12), so these replace that step. */
 #define QGEMM_IN_FP32 0
 #define QGEMM_IN_BF16 1
 
