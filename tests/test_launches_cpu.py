@@ -213,8 +213,10 @@ x, c, s, rows = far(0), far(10), far(20), (1 << 29) + 64    # K = 32, shuffled: 
 for fn, row in ((L.qgemm_quant_mxfp8, 32), (L.qgemm_quant_mxfp4, 16)):
     stub.stub_reset(0)
     st = fn(P(x), 1, rows, 32, 32, P(c), row, P(s), 1, 1, None)
-    _, gx, gy, gz, threads, _ = launches()[0]
-    print(st == 0 and threads == 256 and gx * threads < 1 << 32 and rows // 32 <= gx * gy * gz < rows // 32 + gy)
+    got = launches()
+    fits = all(g[1] * 256 < 1 << 32 and g[2:5] == (1, 1, 256) for g in got)
+    # (the 96 rows left take 8 rows a workgroup)
+    print(st == 0 and fits and [g[1] for g in got] == [(1 << 24) - 1, 12])
 """
 
 
