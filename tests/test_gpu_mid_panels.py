@@ -55,7 +55,8 @@ def _run(qgemm, kind, a, b, sa, sb, m, n, k, out_dtype, extra, split):
 
 
 # K-tiles: below, at and past the ring's four stages and a panel, an odd
-# count (no panels), and 40 (split: slices that start inside a panel)
+# count (no panels), and 40 and 44 (split: in slices of eight, and of nine,
+# which start inside a panel)
 @pytest.mark.parametrize("ktiles,m,n,split", [(1, 130, 70, False), (2, 65, 130, False), (3, 70, 200, False),
                                               (4, 129, 129, False), (5, 200, 100, False), (8, 100, 300, False),
                                               (12, 70, 70, False), (40, 150, 260, True), (44, 300, 1500, True),
